@@ -1724,7 +1724,7 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
             BatchArgs b{};
             b.emb16 = g.emb16; b.n = n_live; b.d = g.d; b.qh = c.bq; b.q = Qt; b.tq = c.btq; b.ts = g.ts;
             b.mods = g.mods; b.lambda = Qg > 0 ? lambda : 0.0f; b.mod_filter = Qg > 0 ? cfg->modality_filter : -1;
-            b.k = kMultiCand; b.q_plain = Qg; b.self_base = knn_count > 0 ? knn_first : -1; b.part = c.bpart;
+            b.k = kMultiCand; b.nrm = g.nrm; b.q_plain = Qg; b.self_base = knn_count > 0 ? knn_first : -1; b.part = c.bpart;
             b.rows_per_range = rpr; b.n_rranges = nrr; b.n_qblocks = nqb;
             b.uniform_tq = (Qg == 0 || std::all_of(h_tq, h_tq + Qg, [&](float x) { return x == h_tq[0]; })) ? 1 : 0;
             MARS_TRY(launch_batch_topk(b, kMultiCand, c.bout, s));
@@ -1990,7 +1990,7 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
             const int32_t q = int32_t(std::min<int64_t>(kChunk, nb - q0));
             BatchArgs a{};
             a.emb16 = g.emb16 + r0 * g.d; a.n = nb; a.d = g.d; a.qh = g.emb16 + (r0 + q0) * g.d; a.q = q; a.tq = tq;
-            a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.q_plain = 0; a.self_base = q0;
+            a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
             a.part = part; a.uniform_tq = 1;
             a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = (q + 63) / 64;
             rc = launch_batch_topk(a, kCand, cand, s);
@@ -2060,7 +2060,7 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
         const int32_t q = int32_t(std::min<int64_t>(kChunk, int64_t(first) + count - q0));
         BatchArgs a{};
         a.emb16 = g.emb16; a.n = n; a.d = g.d; a.qh = g.emb16 + q0 * g.d; a.q = q; a.tq = tq;
-        a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.q_plain = 0; a.self_base = q0;
+        a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
         a.part = part; a.uniform_tq = 1;
         a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = (q + 63) / 64;
         rc = launch_batch_topk(a, kCand, cand, s);

@@ -121,25 +121,28 @@ void k_batch_mm(BatchArgs a) {
     }
     // The loads of stage st of tile `tile` (st >= NS: stage st - NS of the next tile; tiles
     // past the last load the last one again) into query buffer bq / corpus buffer bc.
-    auto issue_q = [&](int tile, int st, int bq) {
+    auto issue_q1 = [&](int tile, int st, int bq, int j) {
         if (st >= NS) { ++tile; st -= NS; }
         const char* const qb = uniform_ptr(reinterpret_cast<const char*>(a.qh) + st * kMK * 2);
-#pragma unroll
-        for (int j = 0; j < kMDma; ++j)
-            __builtin_amdgcn_global_load_lds(qb + qoff[j], &sh.q[bq][(wave * kMDma + j) * 64], 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(qb + qoff[j], &sh.q[bq][(wave * kMDma + j) * 64], 16, 0, 0);
     };
-    auto issue_c = [&](int tile, int st, int bc) {
+    auto issue_c1 = [&](int tile, int st, int bc, int j) {
         if (st >= NS) { ++tile; st -= NS; }
         tile = tile < int(ntiles) ? tile : int(ntiles) - 1;
         const int64_t trow = r0 + int64_t(tile) * kMR;
         const char* const tb = uniform_ptr(reinterpret_cast<const char*>(a.emb16 + trow * d) + st * kMK * 2);
         const uint32_t last = uint32_t(r1 - 1 - trow < kMR - 1 ? r1 - 1 - trow : kMR - 1);   // rows past r1 - 1 clamp
+        const uint32_t rl = uint32_t(srow + 16 * j) < last ? uint32_t(srow + 16 * j) : last;
+        __builtin_amdgcn_global_load_lds(tb + (rl * uint32_t(d * 2) + uint32_t(spiece * 16)),
+                                         &sh.e[bc][(wave * kMDma + j) * 64], 16, 0, 0);
+    };
+    auto issue_q = [&](int tile, int st, int bq) {
 #pragma unroll
-        for (int j = 0; j < kMDma; ++j) {
-            const uint32_t rl = uint32_t(srow + 16 * j) < last ? uint32_t(srow + 16 * j) : last;
-            __builtin_amdgcn_global_load_lds(tb + (rl * uint32_t(d * 2) + uint32_t(spiece * 16)),
-                                             &sh.e[bc][(wave * kMDma + j) * 64], 16, 0, 0);
-        }
+        for (int j = 0; j < kMDma; ++j) issue_q1(tile, st, bq, j);
+    };
+    auto issue_c = [&](int tile, int st, int bc) {
+#pragma unroll
+        for (int j = 0; j < kMDma; ++j) issue_c1(tile, st, bc, j);
     };
 
     uint64_t list[K];                              // query q0 + tid
@@ -175,20 +178,29 @@ void k_batch_mm(BatchArgs a) {
 
     f32x16 acc[4][4];
     f16x8 fa0[4], fb0[4], fa1[4], fb1[4];          // fragments of k-step 0 / 1 of a stage
-    auto read_frags = [&](int bc, int bq, int kk, f16x8 (&af)[4], f16x8 (&bf)[4]) {
+    // read i of a k-step's eight fragment reads, in the order the MFMAs need them
+    auto read_frag = [&](int bc, int bq, int kk, int i, f16x8 (&af)[4], f16x8 (&bf)[4]) {
         const int pc = (2 * kk + lh) ^ ((lm >> 2) & 3);        // swizzled slot of this lane's piece
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
+        if (i == 0 || i >= 5) {
+            const int x = i == 0 ? 0 : i - 4;
             af[x] = __builtin_bit_cast(f16x8, sh.e[bc][(wr * 128 + x * 32 + lm) * 4 + pc]);
-            bf[x] = __builtin_bit_cast(f16x8, sh.q[bq][(wq * 128 + x * 32 + lm) * 4 + pc]);
+        } else {
+            bf[i - 1] = __builtin_bit_cast(f16x8, sh.q[bq][(wq * 128 + (i - 1) * 32 + lm) * 4 + pc]);
         }
     };
-    auto mma = [&](const f16x8 (&af)[4], const f16x8 (&bf)[4]) {
+    auto read_frags = [&](int bc, int bq, int kk, f16x8 (&af)[4], f16x8 (&bf)[4]) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int i = 0; i < 8; ++i) read_frag(bc, bq, kk, i, af, bf);
+    };
+    // one k-step's 16 MFMAs with a piece of other work (LDS reads, stage loads) after each
+    auto mma = [&](const f16x8 (&af)[4], const f16x8 (&bf)[4], auto&& between) {
 #pragma unroll
-            for (int qt = 0; qt < 4; ++qt)
-                acc[rt][qt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[rt], bf[qt], acc[rt][qt], 0, 0, 0);
+        for (int i = 0; i < 16; ++i) {
+            acc[i >> 2][i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i >> 2], bf[i & 3], acc[i >> 2][i & 3], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            between(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
 
     // Selection staging: a chunk's raw scores as [query][row] fp32, queries 0 .. 127 in the
@@ -201,15 +213,23 @@ void k_batch_mm(BatchArgs a) {
     float* wbase = nullptr;                                         // this wave's 128 queries
     const float* obase = nullptr;
     const int oswz = (tid >> 1) & 7;
+    // No dot can be NaN (or infinite): |dot| and every partial sum of it are at most the
+    // squared largest row norm, up to rounding (the queries are rows). False for rows with
+    // NaN or infinities, and where the norms are not known.
+    bool nan_free = false;
+    if (a.nrm != nullptr) {
+        const float e16 = __uint_as_float(a.nrm[1]);
+        nan_free = e16 < 1e15f;
+    }
     // The owner's threshold for the next tile: the larger of its floor and, once its list is
-    // full, its K-th score; a dot below it cannot enter the list. Without either the wave's
-    // tiles go the full way. Queries past the batch offer nothing.
+    // full, its K-th score; a dot below it cannot enter the list. Without either, or where
+    // dots may be NaN, the wave's tiles go the full way. Queries past the batch offer nothing.
     auto publish = [&]() {
         float th = INFINITY;
         bool ok = true;
         if (my_q < a.q) {
             th = fmaxf(list[K - 1] != kEmptyKey ? key_score(list[K - 1]) : -INFINITY, my_floor);
-            ok = th > -INFINITY;
+            ok = th > -INFINITY && nan_free;
         }
         int ut = tid;
         asm volatile("" : "+v"(ut));
@@ -329,32 +349,39 @@ void k_batch_mm(BatchArgs a) {
         lds_barrier();
         read_frags(bc, bq, 0, fa0, fb0);
         // Stage st, with its k-step-0 fragments already read:
-        //   read k-step 1; MFMAs of k-step 0 (the reads land meanwhile);
+        //   MFMAs of k-step 0, the reads of k-step 1 between them;
         //   wait for stage st + 1's loads and meet: every wave's loads of st + 1 landed,
-        //   every wave is done reading stage st; refill stage st's buffers with the queries
-        //   of stage st + kMBQ and the rows of stage st + kMBC (the tile's last stage leaves
-        //   that to after the selection, which needs the buffers); read k-step 0 of st + 1;
-        //   MFMAs of k-step 1 (the reads land meanwhile).
-        // (sched_barrier keeps each block of reads ahead of the MFMAs it overlaps: the
-        // scheduler would otherwise sink the reads next to their uses. Unrolled whole: a
-        // full pass of the 1M k-NN chunk took 1.72 ms against 1.76 ms unrolled by 4 on one
-        // box; by 4 against by 2, 1.79 against 1.82 ms on another.)
+        //   every wave is done reading stage st;
+        //   MFMAs of k-step 1; between them the reads of st + 1's k-step 0, and the loads
+        //   that refill stage st's buffers with the queries of stage st + kMBQ and the rows
+        //   of stage st + kMBC (the tile's last stage leaves those to after the selection,
+        //   which needs the buffers).
+        // The fragment reads and the stage loads go between the MFMAs, one or two after each:
+        // a wave that issues its eight loads at once waits for the address unit (16 cycles
+        // per load, four waves at it) with its matrix core idle. 8 chunks of 1024 queries
+        // over 1M rows: 14.88 ms with the loads and reads in blocks, 14.39 ms so.
+        // (sched_barrier pins them there. Unrolled whole: a full pass of the 1M k-NN chunk
+        // took 1.72 ms against 1.76 ms unrolled by 4 on one box; by 4 against by 2, 1.79
+        // against 1.82 ms on another.)
 #pragma unroll
         for (int st = 0; st < NS; ++st) {
-            read_frags(bc, bq, 1, fa1, fb1);
-            __builtin_amdgcn_sched_barrier(0);
-            mma(fa0, fb0);
+            mma(fa0, fb0, [&](int i) {
+                if (i < 8) read_frag(bc, bq, 1, i, fa1, fb1);
+            });
             if (st + 1 < NS) {
                 __builtin_amdgcn_s_waitcnt(wait_vm(kStageWait));
                 lds_barrier();
-                issue_q(int(t), st + kMBQ, bq);
-                issue_c(int(t), st + kMBC, bc);
+                const int oc = bc, oq = bq;
                 bc = bc + 1 == kMBC ? 0 : bc + 1;
                 bq = (bq + 1) & (kMBQ - 1);
-                read_frags(bc, bq, 0, fa0, fb0);
-                __builtin_amdgcn_sched_barrier(0);
+                mma(fa1, fb1, [&](int i) {
+                    if (i < 8) read_frag(bc, bq, 0, i, fa0, fb0);
+                    if ((i & 1) == 0 && i < 8) issue_q1(int(t), st + kMBQ, oq, i >> 1);
+                    if ((i & 1) == 0 && i >= 8) issue_c1(int(t), st + kMBC, oc, (i - 8) >> 1);
+                });
+            } else {
+                mma(fa1, fb1, [&](int) {});
             }
-            mma(fa1, fb1);
         }
         // every wave is done with the tile's last stage's buffers (bc, bq): the selection's
         // LDS until the deferred loads refill them
@@ -371,9 +398,10 @@ void k_batch_mm(BatchArgs a) {
         if (!sample && !full_way) {
             // Slot selection, in three steps.
             // 1. Each lane tests its 16 dots of each 32 x 32 block at once: their maximum
-            //    (NaN ignored) against the query's threshold, and their sum, NaN when a dot
-            //    is NaN (offered, as the full way offers NaN). A lane that reaches it appends
-            //    the block's 16 dots to its wave's records (ballot compaction).
+            //    against the query's threshold (fmaxf drops NaN, so this way is taken only
+            //    where no dot can be NaN; summing the dots to find one took 42 us more per
+            //    1M-row chunk of 1024 queries, 2.5% of its full pass). A lane that reaches it
+            //    appends the block's 16 dots to its wave's records (ballot compaction).
             // 2. The wave's lanes take one record each and offer every dot not below the
             //    threshold: a slot index from the query's counter, then (row, dot).
             // 3. The owners insert their candidates.
@@ -387,16 +415,13 @@ void k_batch_mm(BatchArgs a) {
             uint2* const slots = reinterpret_cast<uint2*>(&sh.q[bq][0]);
             const uint32_t rowb = uint32_t(wr * 128 + 4 * (ul >> 5));
             uint32_t nrec = 0;                                          // uniform
-            // whether a lane's 16 dots of a block can reach threshold th: their maximum (NaN
-            // ignored) is not below it, or their sum is NaN (a NaN dot), as trees
+            // whether a lane's 16 dots of a block can reach threshold th: their maximum is not
+            // below it
             auto block_hit = [](const f32x16& xv, float th) {
                 const float m = fmaxf(fmaxf(fmaxf(fmaxf(xv[0], xv[1]), xv[2]), fmaxf(fmaxf(xv[3], xv[4]), xv[5])),
                                       fmaxf(fmaxf(fmaxf(xv[6], xv[7]), xv[8]), fmaxf(fmaxf(xv[9], xv[10]), xv[11])));
                 const float m2 = fmaxf(fmaxf(fmaxf(xv[12], xv[13]), xv[14]), xv[15]);
-                const float s0 = (xv[0] + xv[1]) + (xv[2] + xv[3]), s1 = (xv[4] + xv[5]) + (xv[6] + xv[7]);
-                const float s2 = (xv[8] + xv[9]) + (xv[10] + xv[11]), s3 = (xv[12] + xv[13]) + (xv[14] + xv[15]);
-                const float sum = (s0 + s1) + (s2 + s3);
-                return !(fmaxf(m, m2) < th) || sum != sum;
+                return !(fmaxf(m, m2) < th);
             };
             // append the block of the lanes that hit to the wave's records
             auto put_records = [&](const f32x16& xv, bool hit, uint64_t hb, int ql, int rt) {

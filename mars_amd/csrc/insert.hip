@@ -316,7 +316,7 @@ int insert_knn_fp16(Graph& g, int64_t first, int32_t nq, int64_t n, int32_t k, h
         BatchArgs a{};
         a.emb16 = g.emb16; a.n = n; a.d = g.d; a.qh = g.emb16 + (first + c0) * g.d; a.q = q; a.tq = g.ins_tq;
         a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kKnnCand;
-        a.q_plain = 0; a.self_base = first + c0; a.part = g.ins_part; a.rows_per_range = rpr; a.n_rranges = nrr;
+        a.nrm = g.nrm; a.q_plain = 0; a.self_base = first + c0; a.part = g.ins_part; a.rows_per_range = rpr; a.n_rranges = nrr;
         a.n_qblocks = nqb; a.uniform_tq = 1;
         MARS_TRY(launch_batch_topk(a, kKnnCand, g.ins_cand, s));
         MARS_TRY(launch_knn_rerank(g.emb, first + c0, q, g.d, g.ins_cand, kKnnCand, k, g.ins_nbrs + int64_t(c0) * k, s,

@@ -517,6 +517,7 @@ struct BatchArgs {
                              // no decay, no filter (the rest use lambda / mod_filter / tq)
     int64_t self_base;       // >= 0: neighbour search j (query q_plain + j) is node self_base + j
                              // and never its own neighbour
+    const uint32_t* nrm;     // optional (k_batch_mm): the fp16 copy's row-norm maxima
     uint64_t* part;          // [n_qblocks][n_rranges][64][K] keys
     int64_t rows_per_range;
     int64_t range_stride;    // row range r starts at row r * range_stride (0: rows_per_range)

@@ -124,3 +124,25 @@ def test_blocked_build_counts_only():
             assert np.all((got[2000 * b:2000 * (b + 1)] // 2000) == b)
     finally:
         mars_amd.free_device(dg)
+
+
+def test_blocked_build_offers_nan_dots():
+    """A row with a NaN: every dot with it is NaN, which orders above every score, so the row
+    heads each list of its block and the rest of the list is the block's exact 7-NN."""
+    n, bad = 6000, 1700
+    c = corpus.make_corpus(n, D, seed=19)
+    emb = c.embeddings.copy()
+    emb[bad, 5] = np.nan
+    dg = device_graph(emb, c.modalities, c.timestamps)
+    try:
+        got = mars_amd.graph_knn(dg, 8, block_rows=3000)
+        assert dg.knn_report == (n, 0)                   # NaN bounds certify nothing
+        nodes = np.setdiff1d(np.arange(0, 3000, 13), [bad])
+        assert np.all(got[nodes, 0] == bad)
+        keep = np.setdiff1d(np.arange(3000), [bad])
+        pos = np.searchsorted(keep, nodes)
+        check_lists(c.embeddings[keep], pos, np.searchsorted(keep, got[nodes, 1:]), 7)
+        nodes = np.arange(3000, 6000, 13)                # the other block has no NaN
+        check_lists(c.embeddings[3000:], nodes - 3000, got[nodes] - 3000)
+    finally:
+        mars_amd.free_device(dg)
