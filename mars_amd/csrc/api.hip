@@ -600,6 +600,33 @@ int query_impl(const mars_graph* gh, mars_ctx* ch, const float* h_q, const float
 
 }  // namespace
 
+int32_t mm_ranges(int32_t groups, int64_t tiles) {
+    const int32_t xg = mm_xcd_groups(groups), xr = 8 / xg;
+    // ranges per XCD: at most 32 workgroups on its 32 CUs
+    const int32_t per = std::max(1, 32 / ((groups + xg - 1) / xg));
+    const int64_t most = std::min<int64_t>(int64_t(per) * xr, std::max<int64_t>(tiles, 1));
+    const int64_t longest = (tiles + most - 1) / most;         // tiles of the longest range
+    return int32_t(std::max<int64_t>(1, (tiles + longest - 1) / std::max<int64_t>(longest, 1)));
+}
+
+int32_t mm_chunk(int64_t q, int64_t n) {
+    const int64_t tiles = (n + 255) / 256;
+    auto steps = [&](int64_t chunk) {                          // tile steps of all launches, one more for each launch
+        int64_t sum = 0;
+        for (int64_t left = q; left > 0; left -= chunk) {
+            const int32_t groups = int32_t((std::min(left, chunk) + 255) / 256);
+            const int64_t rr = mm_ranges(groups, tiles);
+            const int64_t same = left >= 2 * chunk ? left / chunk - 1 : 1;   // equal launches counted at once
+            sum += ((tiles + rr - 1) / rr + 1) * same;
+            left -= (same - 1) * chunk;
+        }
+        return sum;
+    };
+    const int64_t launches = (q + kMmMaxQ - 1) / kMmMaxQ;
+    const int64_t even = std::max<int64_t>(256, ((q + launches - 1) / launches + 255) / 256 * 256);
+    return int32_t(steps(8192) < steps(even) ? 8192 : even);
+}
+
 // Row ranges x query blocks for the batched scan: one 512-thread workgroup per CU
 // (256 CUs), all query blocks of a row range on one XCD.
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
@@ -612,6 +639,7 @@ void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n
     const int64_t align = gemm ? 256 : 16;                            // rows per tile
     int32_t rr = std::max(8, (256 / std::max(tiles, 1)) / 8 * 8);
     const int64_t max_rr = std::max<int64_t>(1, (n + align - 1) / align);   // at least one tile per range
+    if (gemm) rr = mm_ranges(tiles, max_rr);
     if (rr > max_ranges) rr = std::max(1, max_ranges);
     if (rr > max_rr) rr = int32_t(max_rr);
     *n_qblocks = qblocks;
@@ -1954,16 +1982,15 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
     MARS_CHECK(g.emb16 != nullptr, MARS_ERR_UNSUPPORTED, "k-NN reads the fp16 corpus: enable it first");
     MARS_CHECK(batch_dim_supported(g.d), MARS_ERR_UNSUPPORTED, "k-NN: embedding_dim %d unsupported", g.d);
     MARS_TRY(use_device(g.device));
-    constexpr int32_t kChunk = 1024;                 // queries per launch (16 query blocks)
     constexpr int32_t kCand = 16;
     const int64_t B = std::min<int64_t>(block_rows, g.n);
+    const int32_t chunk = mm_chunk(B, B);            // queries per launch
     // nodes [lo, hi): the requested blocks
     const int64_t lo = std::min<int64_t>(int64_t(first_block) * block_rows, g.n);
     const int64_t hi = std::min<int64_t>(lo + int64_t(n_blocks) * block_rows, g.n);
     if (hi <= lo) return MARS_OK;
     int32_t nrr = 0, nqb = 0;
     int64_t rpr = 0;
-    batch_grid(B, kChunk, true, &nrr, &nqb, &rpr);   // the largest block sizes the scratch
     float* tq = nullptr; uint64_t* part = nullptr; uint64_t* cand = nullptr; int32_t* dn = nullptr;
     int32_t* cert = nullptr;
     hipStream_t s = nullptr;
@@ -1972,27 +1999,28 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
         dfree(tq); dfree(part); dfree(cand); dfree(dn); dfree(cert);
         if (s) (void)hipStreamDestroy(s);
     };
-    if ((rc = dmalloc(&tq, kChunk)) || (rc = dmalloc(&part, size_t(nqb) * nrr * 64 * kCand)) ||
-        (rc = dmalloc(&cand, size_t(kChunk) * kCand)) || (rc = dmalloc(&dn, size_t(hi - lo) * k)) ||
+    // (a launch of any size has at most 256 x 256 queries x row ranges)
+    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(kMaxRangeQueries) * kCand)) ||
+        (rc = dmalloc(&cand, size_t(chunk) * kCand)) || (rc = dmalloc(&dn, size_t(hi - lo) * k)) ||
         (rc = dmalloc(&cert, size_t(hi - lo)))) {
         cleanup();
         return rc;
     }
     hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMemsetAsync(tq, 0, kChunk * sizeof(float), s);
+    if (e == hipSuccess) e = hipMemsetAsync(tq, 0, size_t(chunk) * sizeof(float), s);
     if (e == hipSuccess) e = hipMemsetAsync(cert, 0, size_t(hi - lo) * sizeof(int32_t), s);
     if (e != hipSuccess) { cleanup(); return set_error(MARS_ERR_HIP, "k-NN setup: %s", hipGetErrorString(e)); }
     // block [r0, r1): rows, queries and candidate ids relative to r0
     for (int64_t r0 = lo; r0 < hi && rc == MARS_OK; r0 += B) {
         const int64_t nb = std::min<int64_t>(B, g.n - r0);
-        batch_grid(nb, kChunk, true, &nrr, &nqb, &rpr);
-        for (int64_t q0 = 0; q0 < nb && rc == MARS_OK; q0 += kChunk) {
-            const int32_t q = int32_t(std::min<int64_t>(kChunk, nb - q0));
+        for (int64_t q0 = 0; q0 < nb && rc == MARS_OK; q0 += chunk) {
+            const int32_t q = int32_t(std::min<int64_t>(chunk, nb - q0));
+            batch_grid(nb, q, true, &nrr, &nqb, &rpr);
             BatchArgs a{};
             a.emb16 = g.emb16 + r0 * g.d; a.n = nb; a.d = g.d; a.qh = g.emb16 + (r0 + q0) * g.d; a.q = q; a.tq = tq;
             a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
             a.part = part; a.uniform_tq = 1;
-            a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = (q + 63) / 64;
+            a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
             rc = launch_batch_topk(a, kCand, cand, s);
             if (rc == MARS_OK)
                 rc = launch_knn_rerank(g.emb + r0 * g.d, q0, q, g.d, cand, kCand, k, dn + (r0 - lo + q0) * k, s,
@@ -2031,12 +2059,11 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
                (long long)first + count, g.n);
     if (count == 0) return MARS_OK;
     MARS_TRY(use_device(g.device));
-    constexpr int32_t kChunk = 1024;                 // queries per launch
     constexpr int32_t kCand = 16;
     const int64_t n = g.n;
+    const int32_t chunk = mm_chunk(count, n);        // queries per launch
     int32_t nrr = 0, nqb = 0;
     int64_t rpr = 0;
-    batch_grid(n, kChunk, true, &nrr, &nqb, &rpr);
     float* tq = nullptr; uint64_t* part = nullptr; uint64_t* cand = nullptr; int32_t* dn = nullptr;
     int32_t* cert = nullptr;
     hipStream_t s = nullptr;
@@ -2045,24 +2072,26 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
         dfree(tq); dfree(part); dfree(cand); dfree(dn); dfree(cert);
         if (s) (void)hipStreamDestroy(s);
     };
-    if ((rc = dmalloc(&tq, kChunk)) || (rc = dmalloc(&part, size_t(nqb) * nrr * 64 * kCand)) ||
-        (rc = dmalloc(&cand, size_t(kChunk) * kCand)) || (rc = dmalloc(&dn, size_t(count) * k)) ||
+    // (a launch of any size has at most 256 x 256 queries x row ranges)
+    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(kMaxRangeQueries) * kCand)) ||
+        (rc = dmalloc(&cand, size_t(chunk) * kCand)) || (rc = dmalloc(&dn, size_t(count) * k)) ||
         (rc = dmalloc(&cert, size_t(count)))) {
         cleanup();
         return rc;
     }
     hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMemsetAsync(tq, 0, kChunk * sizeof(float), s);
+    if (e == hipSuccess) e = hipMemsetAsync(tq, 0, size_t(chunk) * sizeof(float), s);
     if (e == hipSuccess) e = hipMemsetAsync(cert, 0, size_t(count) * sizeof(int32_t), s);
     if (e != hipSuccess) { cleanup(); return set_error(MARS_ERR_HIP, "k-NN range setup: %s", hipGetErrorString(e)); }
     // queries [q0, q0 + q) against every node; the query's own id is excluded
-    for (int64_t q0 = first; q0 < int64_t(first) + count && rc == MARS_OK; q0 += kChunk) {
-        const int32_t q = int32_t(std::min<int64_t>(kChunk, int64_t(first) + count - q0));
+    for (int64_t q0 = first; q0 < int64_t(first) + count && rc == MARS_OK; q0 += chunk) {
+        const int32_t q = int32_t(std::min<int64_t>(chunk, int64_t(first) + count - q0));
+        batch_grid(n, q, true, &nrr, &nqb, &rpr);
         BatchArgs a{};
         a.emb16 = g.emb16; a.n = n; a.d = g.d; a.qh = g.emb16 + q0 * g.d; a.q = q; a.tq = tq;
         a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
         a.part = part; a.uniform_tq = 1;
-        a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = (q + 63) / 64;
+        a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
         rc = launch_batch_topk(a, kCand, cand, s);
         if (rc == MARS_OK)
             rc = launch_knn_rerank(g.emb, q0, q, g.d, cand, kCand, k, dn + (q0 - first) * k, s, g.nrm,

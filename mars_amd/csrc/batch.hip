@@ -222,27 +222,30 @@ __global__ __launch_bounds__(kBWaves * 64) void k_batch_scan(BatchArgs a) {
     }
 }
 
-// One workgroup of eight waves per query: merge n_rranges lists of K keys into the best
-// k_out. Each wave takes every eighth round of 8 x 64 keys (loads in flight together; a
-// chunk with many keys under the wave's bound is sorted and merged in registers, one with
-// a few inserts them one by one), then wave 0 merges the eight lists. (One wave per
-// query, inserting every key under its bound one at a time: 21 us for 256 queries of
-// 4,096 keys; this form: 13 us.)
+// Merge n_rranges lists of K keys per query into the best k_out, W waves per query. Each wave
+// takes every W-th round of 8 x 64 keys (loads in flight together; a chunk with many keys
+// under the wave's bound is sorted and merged in registers, one with a few inserts them one
+// by one), then the query's first wave merges the W lists. W = 8, a workgroup per query, for
+// many ranges (256 queries of 4,096 keys: 13 us; one wave per query, every key under its bound
+// inserted one at a time: 21 us). W = 1, four queries per workgroup, where one round holds
+// all of a query's keys: the other seven waves would have none.
 constexpr int kMergeWaves = 8;
+constexpr int kMergeLd = 8;
 constexpr int kRerankPieces = 3;  // k_knn_rerank: 16-byte pieces per lane and row (d <= 768)
-__global__ __launch_bounds__(kMergeWaves * 64) void k_batch_merge(const uint64_t* __restrict__ part, int32_t n_rranges,
-                                                                  int32_t kpart, int32_t q, int32_t k_out,
-                                                                  uint64_t* __restrict__ out) {
-    __shared__ uint64_t s_l[kMergeWaves][64];
-    const int lane = int(threadIdx.x & 63u), wave = int(threadIdx.x >> 6);
-    const int qi = int(blockIdx.x);
-    if (qi >= q) return;                               // the whole workgroup
+template <int W>
+__global__ __launch_bounds__(W == 1 ? 256 : W * 64) void k_batch_merge(const uint64_t* __restrict__ part,
+                                                                      int32_t n_rranges, int32_t kpart, int32_t q,
+                                                                      int32_t k_out, uint64_t* __restrict__ out) {
+    __shared__ uint64_t s_l[W][64];
+    const int lane = int(threadIdx.x & 63u), w0 = int(threadIdx.x >> 6);
+    const int wave = W == 1 ? 0 : w0;                  // of the query's W
+    const int qi = W == 1 ? int(blockIdx.x) * 4 + w0 : int(blockIdx.x);
+    if (qi >= q) return;                               // the whole workgroup, or (W = 1) the wave
     const int qb = qi / kBQ, j = qi % kBQ;
     uint64_t list = kEmptyKey, thr = kEmptyKey;
     const int total = n_rranges * kpart;
     const int kshift = kpart == 8 ? 3 : 4;             // kpart is 8 or 16 (batch_kpart)
-    constexpr int kMergeLd = 8;
-    for (int base = wave * 64 * kMergeLd; base < total; base += kMergeWaves * 64 * kMergeLd) {
+    for (int base = wave * 64 * kMergeLd; base < total; base += W * 64 * kMergeLd) {
         uint64_t xs[kMergeLd];
 #pragma unroll
         for (int c = 0; c < kMergeLd; ++c) {
@@ -256,13 +259,14 @@ __global__ __launch_bounds__(kMergeWaves * 64) void k_batch_merge(const uint64_t
 #pragma unroll
         for (int c = 0; c < kMergeLd; ++c) wave_offer(list, thr, xs[c], lane, k_out);
     }
-    s_l[wave][lane] = list;
-    __syncthreads();
-    if (wave == 0) {
+    if constexpr (W > 1) {
+        s_l[wave][lane] = list;
+        __syncthreads();
+        if (wave != 0) return;
 #pragma unroll
-        for (int w = 1; w < kMergeWaves; ++w) list = wave_merge64(list, s_l[w][lane], lane, k_out);
-        if (lane < k_out) out[int64_t(qi) * k_out + lane] = list;
+        for (int w = 1; w < W; ++w) list = wave_merge64(list, s_l[w][lane], lane, k_out);
     }
+    if (lane < k_out) out[int64_t(qi) * k_out + lane] = list;
 }
 
 // Exact fp32 rescoring of kc candidates per node; keeps k_out by (score desc, id asc).
@@ -397,7 +401,11 @@ int launch_batch_scan(const BatchArgs& a, hipStream_t s) {
 int launch_batch_merge(const uint64_t* part, int32_t n_rranges, int32_t kpart, int32_t q, int32_t k_out,
                        uint64_t* out, hipStream_t s) {
     MARS_CHECK(kpart == 8 || kpart == 16, MARS_ERR_INVALID, "batched merge: %d keys per range", kpart);
-    MARS_LAUNCH(k_batch_merge, dim3(unsigned(q)), dim3(kMergeWaves * 64), 0, s, part, n_rranges, kpart, q, k_out, out);
+    if (n_rranges * kpart <= 64 * kMergeLd)
+        MARS_LAUNCH((k_batch_merge<1>), dim3(unsigned((q + 3) / 4)), dim3(256), 0, s, part, n_rranges, kpart, q, k_out, out);
+    else
+        MARS_LAUNCH((k_batch_merge<kMergeWaves>), dim3(unsigned(q)), dim3(kMergeWaves * 64), 0, s, part, n_rranges, kpart,
+                    q, k_out, out);
     return MARS_OK;
 }
 
@@ -411,9 +419,11 @@ int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, 
     // The floor pays where a range is long: without it a query inserts about
     // K (1 + ln(rows / K)) rows per range (every new best of the rows seen so far), with
     // it about rows x K / sampled rows.
-    if (a.q > kRqMaxScanQ && a.rows_per_range >= kSampleDiv * kSampleRowsMin) {
+    const bool gemm = batch_uses_gemm(a.q, a.q_plain == 0);
+    if (gemm || (a.q > kRqMaxScanQ && a.rows_per_range >= kSampleDiv * kSampleRowsMin)) {
         BatchArgs b = a;
-        b.rows_per_range = std::min<int64_t>(kSampleRowsMax, a.rows_per_range / kSampleDiv / 16 * 16);
+        b.rows_per_range = gemm ? std::min<int64_t>(a.rows_per_range, (kMmSampleTiles + a.n_rranges - 1) / a.n_rranges * 256)
+                                : std::min<int64_t>(kSampleRowsMax, a.rows_per_range / kSampleDiv / 16 * 16);
         b.range_stride = a.rows_per_range;
         b.sample_pass = 1;
         MARS_TRY(launch_batch_scan(b, s));

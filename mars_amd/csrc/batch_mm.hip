@@ -96,8 +96,17 @@ void k_batch_mm(BatchArgs a) {
     const int wr = wave & 1, wq = wave >> 1;       // row half, query half
     const int lm = lane & 31, lh = lane >> 5;
     constexpr int d = NS * kMK;
-    const int r_id = int(blockIdx.x) % a.n_rranges;
-    const int q0 = (int(blockIdx.x) / a.n_rranges) * kMQ;
+    // XCD x (= blockIdx % 8) takes a block of the (query group, row range) grid: group slice
+    // x % xg of xg, range slice x / xg of 8 / xg, all groups of a range next to each other
+    // (the launch rounds the slices up; workgroups past them leave).
+    const int ngrp = (a.q + kMQ - 1) / kMQ;
+    const int xcd = int(blockIdx.x) & 7, slot = int(blockIdx.x) >> 3;
+    const int xg = mm_xcd_groups(ngrp), xr = 8 / xg;
+    const int gs = ngrp * (xcd % xg) / xg, gn = ngrp * (xcd % xg + 1) / xg - gs;
+    const int rs = a.n_rranges * (xcd / xg) / xr, rn = a.n_rranges * (xcd / xg + 1) / xr - rs;
+    if (slot >= gn * rn) return;                   // the whole workgroup
+    const int r_id = rs + slot / gn;
+    const int q0 = (gs + slot % gn) * kMQ;
     const int64_t r0 = int64_t(r_id) * (a.range_stride > 0 ? a.range_stride : a.rows_per_range);
     const int64_t r1 = (a.n < r0 + a.rows_per_range) ? a.n : r0 + a.rows_per_range;
     const int64_t ntiles = r1 > r0 ? (r1 - r0 + kMR - 1) / kMR : 0;
@@ -544,7 +553,8 @@ void k_batch_mm(BatchArgs a) {
 
 template <int NS, int K>
 int launch_mm_t(const BatchArgs& a, hipStream_t s) {
-    const unsigned grid = unsigned(a.n_rranges * ((a.q + kMQ - 1) / kMQ));
+    const int32_t ngrp = (a.q + kMQ - 1) / kMQ, xg = mm_xcd_groups(ngrp), xr = 8 / xg;
+    const unsigned grid = 8u * unsigned(((ngrp + xg - 1) / xg) * ((a.n_rranges + xr - 1) / xr));
     MARS_LAUNCH((k_batch_mm<NS, K>), dim3(grid), dim3(kMThreads), 0, s, a);
     return MARS_OK;
 }

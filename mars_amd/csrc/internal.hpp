@@ -548,6 +548,29 @@ bool batch_dim_supported(int32_t d);
 // (With 64 queries per workgroup k_batch_rq measured slower than the scan: 445 against
 // 408 us on a random 1M corpus.)
 constexpr int32_t kGemmMinQ = 1024;
+// k_batch_mm's grid: groups of 256 queries x row ranges of 256-row tiles, one workgroup each
+// and one per CU. mm_xcd_groups: the XCDs a launch's groups are split over, the fewest that
+// leave an XCD at most five (five groups' queries, d = 768, are 1.9 MiB of its 4 MiB L2, read
+// again for every tile); the ranges are split over the other factor of 8. mm_ranges: the
+// row ranges of a launch, the number that leaves the longest range shortest with at most 32
+// workgroups on an XCD. A launch takes at most kMmMaxQ queries. (Launches of 1024 queries, each
+// with its own passes, merges and rescoring, against these: the 8-NN graph of 10K rows 1669
+// -> 627 us, where 1024 queries were 160 workgroups of one tile; 8,192 nodes over 1M rows
+// 14.3 -> 11.9 ms, where 8 long ranges instead of 64 leave each query fewer rows that ever
+// enter a list, and one launch one tail.)
+constexpr int32_t kMmMaxQ = 10240;
+__host__ __device__ inline int32_t mm_xcd_groups(int32_t groups) {
+    int32_t xg = 1;
+    while (xg < 8 && (groups + xg - 1) / xg > 5) xg *= 2;
+    return xg;
+}
+int32_t mm_ranges(int32_t groups, int64_t tiles);
+// Queries (rounded up to 64) x row ranges of any launch batch_grid lays out, at most: 256 groups x
+// ranges of 256 queries.
+constexpr int64_t kMaxRangeQueries = 256 * 256;
+// The queries per launch for a build of q queries over n rows: as many as kMmMaxQ in equal
+// launches, or 8192 (32 groups, which fill the chip evenly) when that takes fewer tile steps.
+int32_t mm_chunk(int64_t q, int64_t n);
 constexpr int32_t kRqMaxScanQ = 64;
 bool batch_uses_gemm(int32_t q, bool plain);
 bool batch_uses_rq(int32_t q, bool plain);
@@ -570,6 +593,11 @@ int launch_batch_merge(const uint64_t* part, int32_t n_rranges, int32_t kpart, i
 constexpr int64_t kSampleDiv = 64;
 constexpr int64_t kSampleRowsMin = 32;
 constexpr int64_t kSampleRowsMax = 1024;
+// k_batch_mm samples whole tiles, kMmSampleTiles of them over its ranges at least: a query then has
+// about 16 / kMmSampleTiles dots above its floor per tile, so a wave's 64 records hold those of
+// its quarter tile (about 1024 / kMmSampleTiles). Small corpora are sampled whole: at 10K rows
+// a second product is cheaper than filling 16-entry lists from every tile (the full way).
+constexpr int64_t kMmSampleTiles = 64;
 // `scanned` (optional) is recorded after the full pass, before the final merge.
 int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, hipEvent_t scanned = nullptr);
 // nrm and cert given: cert[node] = 1 when the node's lists are certified exact (k_knn_rerank)

@@ -126,9 +126,10 @@ def test_blocked_build_counts_only():
         mars_amd.free_device(dg)
 
 
-def test_blocked_build_offers_nan_dots():
-    """A row with a NaN: every dot with it is NaN, which orders above every score, so the row
-    heads each list of its block and the rest of the list is the block's exact 7-NN."""
+def test_blocked_build_with_a_nan_row():
+    """A row with a NaN (dots that no threshold test may drop or rank): its block's other lists
+    are exact over the other rows, the row's own list is the block's first ids, the other block
+    is untouched, and nothing is certified."""
     n, bad = 6000, 1700
     c = corpus.make_corpus(n, D, seed=19)
     emb = c.embeddings.copy()
@@ -136,13 +137,31 @@ def test_blocked_build_offers_nan_dots():
     dg = device_graph(emb, c.modalities, c.timestamps)
     try:
         got = mars_amd.graph_knn(dg, 8, block_rows=3000)
-        assert dg.knn_report == (n, 0)                   # NaN bounds certify nothing
+        assert dg.knn_report == (n, 0)
+        assert np.array_equal(got[bad], np.arange(8)) and not np.any(got == bad)
         nodes = np.setdiff1d(np.arange(0, 3000, 13), [bad])
-        assert np.all(got[nodes, 0] == bad)
         keep = np.setdiff1d(np.arange(3000), [bad])
-        pos = np.searchsorted(keep, nodes)
-        check_lists(c.embeddings[keep], pos, np.searchsorted(keep, got[nodes, 1:]), 7)
-        nodes = np.arange(3000, 6000, 13)                # the other block has no NaN
+        check_lists(c.embeddings[keep], np.searchsorted(keep, nodes), np.searchsorted(keep, got[nodes]))
+        nodes = np.arange(3000, 6000, 13)
         check_lists(c.embeddings[3000:], nodes - 3000, got[nodes] - 3000)
+    finally:
+        mars_amd.free_device(dg)
+
+
+# all-pairs sizes around the tile (256), the smallest MFMA build (1024 queries), the group
+# splits over the XCDs (5, 10, 20 and 40 groups), and two launches (10,241); ranges whose
+# groups do not divide evenly
+@pytest.mark.parametrize("n, first, count", [(1024, 0, 0), (1025, 0, 0), (1281, 0, 0), (2561, 0, 0), (5121, 0, 0),
+                                             (10_240, 0, 0), (10_241, 0, 0), (3000, 1400, 1600), (50_001, 7, 2_817),
+                                             (50_001, 44_000, 6_001)])
+def test_build_grids(n, first, count):
+    c = corpus.make_corpus(n, 256, seed=n)
+    dg = device_graph(c.embeddings, c.modalities, c.timestamps)
+    try:
+        got = mars_amd.graph_knn_range(dg, 8, first, count) if count else mars_amd.graph_knn(dg, 8)
+        u, r = dg.knn_report if not count else mars_amd.graph_knn_report(dg)
+        assert r == u and u <= max(4, len(got) // 100)
+        idx = np.unique(np.r_[np.arange(0, len(got), 37), len(got) - 1])
+        check_lists(c.embeddings, first + idx, got[idx])
     finally:
         mars_amd.free_device(dg)
