@@ -630,7 +630,7 @@ int32_t mm_chunk(int64_t q, int64_t n) {
 // Row ranges x query blocks for the batched scan: one 512-thread workgroup per CU
 // (256 CUs), all query blocks of a row range on one XCD.
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
-                int32_t max_ranges) {
+                int32_t max_ranges, int32_t kp) {
     // n_qblocks counts 64-query blocks (the layout of the partial keys) for every kernel
     const int32_t qblocks = (q + 63) / 64;
     const bool gemm = batch_uses_gemm(q, plain), rq = batch_uses_rq(q, plain);
@@ -644,6 +644,7 @@ void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n
     if (rr > max_rr) rr = int32_t(max_rr);
     *n_qblocks = qblocks;
     *rows_per_range = ((n + rr - 1) / rr + align - 1) / align * align;
+    if (rq && kp > 0 && *rows_per_range < kRqFloorTiles * align) *rows_per_range = kp;
     *n_rranges = int32_t((n + *rows_per_range - 1) / *rows_per_range);
 }
 
@@ -1550,8 +1551,8 @@ int mars_query_batch(const mars_graph* gh, mars_ctx* ch, const float* dq, int32_
     const int32_t n_live = __atomic_load_n(&g.n, __ATOMIC_ACQUIRE);
     int32_t nrr = 0, nqb = 0;
     int64_t rpr = 0;
-    batch_grid(n_live, Q, false, &nrr, &nqb, &rpr);
     const int32_t kp = batch_kpart(K);
+    batch_grid(n_live, Q, false, &nrr, &nqb, &rpr, 256, kp);
     MARS_TRY(ensure_batch_scratch(c, Q, int64_t(nqb) * nrr * 64 * kp));
     hipStream_t s = c.stream;
     MARS_HIP(hipMemcpyAsync(c.btq, h_tq, size_t(Q) * sizeof(float), hipMemcpyHostToDevice, s));
@@ -1737,8 +1738,8 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
         } else {
             int32_t nrr = 0, nqb = 0;
             int64_t rpr = 0;
-            batch_grid(n_live, Qt, Qg == 0, &nrr, &nqb, &rpr);   // the k-NN queries alone: plain
             const int32_t kp = batch_kpart(kMultiCand);
+            batch_grid(n_live, Qt, Qg == 0, &nrr, &nqb, &rpr, 256, kp);   // the k-NN queries alone: plain
             MARS_TRY(ensure_batch_scratch(c, Qt, int64_t(nqb) * nrr * 64 * kp));
             if (Qg > 0) {
                 MARS_HIP(hipMemcpyAsync(c.btq, h_tq, size_t(Qg) * sizeof(float), hipMemcpyHostToDevice, s));
@@ -1991,6 +1992,14 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
     if (hi <= lo) return MARS_OK;
     int32_t nrr = 0, nqb = 0;
     int64_t rpr = 0;
+    int64_t part_keys = 0;                           // the largest launch's
+    for (const int64_t nb : {B, (hi - lo) % B}) {
+        for (const int64_t q : {std::min<int64_t>(chunk, nb), nb % chunk}) {
+            if (q == 0) continue;
+            batch_grid(nb, int32_t(q), true, &nrr, &nqb, &rpr, 256, kCand);
+            part_keys = std::max(part_keys, int64_t(nqb) * nrr * 64 * kCand);
+        }
+    }
     float* tq = nullptr; uint64_t* part = nullptr; uint64_t* cand = nullptr; int32_t* dn = nullptr;
     int32_t* cert = nullptr;
     hipStream_t s = nullptr;
@@ -1999,8 +2008,7 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
         dfree(tq); dfree(part); dfree(cand); dfree(dn); dfree(cert);
         if (s) (void)hipStreamDestroy(s);
     };
-    // (a launch of any size has at most 256 x 256 queries x row ranges)
-    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(kMaxRangeQueries) * kCand)) ||
+    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(part_keys))) ||
         (rc = dmalloc(&cand, size_t(chunk) * kCand)) || (rc = dmalloc(&dn, size_t(hi - lo) * k)) ||
         (rc = dmalloc(&cert, size_t(hi - lo)))) {
         cleanup();
@@ -2015,7 +2023,7 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
         const int64_t nb = std::min<int64_t>(B, g.n - r0);
         for (int64_t q0 = 0; q0 < nb && rc == MARS_OK; q0 += chunk) {
             const int32_t q = int32_t(std::min<int64_t>(chunk, nb - q0));
-            batch_grid(nb, q, true, &nrr, &nqb, &rpr);
+            batch_grid(nb, q, true, &nrr, &nqb, &rpr, 256, kCand);
             BatchArgs a{};
             a.emb16 = g.emb16 + r0 * g.d; a.n = nb; a.d = g.d; a.qh = g.emb16 + (r0 + q0) * g.d; a.q = q; a.tq = tq;
             a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
@@ -2064,6 +2072,12 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
     const int32_t chunk = mm_chunk(count, n);        // queries per launch
     int32_t nrr = 0, nqb = 0;
     int64_t rpr = 0;
+    int64_t part_keys = 0;                           // the largest launch's
+    for (const int64_t q : {std::min<int64_t>(chunk, count), int64_t(count % chunk)}) {
+        if (q == 0) continue;
+        batch_grid(n, int32_t(q), true, &nrr, &nqb, &rpr, 256, kCand);
+        part_keys = std::max(part_keys, int64_t(nqb) * nrr * 64 * kCand);
+    }
     float* tq = nullptr; uint64_t* part = nullptr; uint64_t* cand = nullptr; int32_t* dn = nullptr;
     int32_t* cert = nullptr;
     hipStream_t s = nullptr;
@@ -2072,8 +2086,7 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
         dfree(tq); dfree(part); dfree(cand); dfree(dn); dfree(cert);
         if (s) (void)hipStreamDestroy(s);
     };
-    // (a launch of any size has at most 256 x 256 queries x row ranges)
-    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(kMaxRangeQueries) * kCand)) ||
+    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(part_keys))) ||
         (rc = dmalloc(&cand, size_t(chunk) * kCand)) || (rc = dmalloc(&dn, size_t(count) * k)) ||
         (rc = dmalloc(&cert, size_t(count)))) {
         cleanup();
@@ -2086,7 +2099,7 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
     // queries [q0, q0 + q) against every node; the query's own id is excluded
     for (int64_t q0 = first; q0 < int64_t(first) + count && rc == MARS_OK; q0 += chunk) {
         const int32_t q = int32_t(std::min<int64_t>(chunk, int64_t(first) + count - q0));
-        batch_grid(n, q, true, &nrr, &nqb, &rpr);
+        batch_grid(n, q, true, &nrr, &nqb, &rpr, 256, kCand);
         BatchArgs a{};
         a.emb16 = g.emb16; a.n = n; a.d = g.d; a.qh = g.emb16 + q0 * g.d; a.q = q; a.tq = tq;
         a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;

@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 
 namespace mars {
 namespace {
@@ -389,6 +390,9 @@ int launch_batch_k(const BatchArgs& a, hipStream_t s) {
 bool batch_dim_supported(int32_t d) { return d == 256 || d == 384 || d == 512 || d == 768; }
 bool batch_uses_gemm(int32_t q, bool plain) { return plain && q >= kGemmMinQ; }
 bool batch_uses_rq(int32_t q, bool plain) { return q > kRqMaxScanQ && !batch_uses_gemm(q, plain); }
+bool batch_keeps_all(int32_t q, bool plain, int64_t rows_per_range, int32_t kp) {
+    return batch_uses_rq(q, plain) && rows_per_range == kp;
+}
 int batch_rq_tiles(int32_t q) { return q <= 128 ? 2 : 4; }
 int batch_kpart(int32_t k) { return k <= 8 ? 8 : 16; }
 
@@ -409,6 +413,23 @@ int launch_batch_merge(const uint64_t* part, int32_t n_rranges, int32_t kpart, i
     return MARS_OK;
 }
 
+namespace {
+
+// The rows of each range that k_batch_rq's sampled pass covers (0: no sampled pass). A pass over s
+// of a range's T tiles costs s tiles; without it a query meets about kp T / s rows per range and
+// nrr ranges that reach its floor, so a wave's 16 QT queries cost kRqHitTiles x 16 QT kp T / (s nrr)
+// tiles: least at the s below. (A pair's selection against a tile's loads, MFMAs and test: about
+// 1 / 20.)
+constexpr double kRqHitTiles = 1.0 / 20;
+int64_t rq_sample_rows(const BatchArgs& a, int32_t kp) {
+    const int64_t tiles = a.rows_per_range / 16;
+    if (tiles < kRqFloorTiles) return 0;
+    const double s = std::sqrt(kRqHitTiles * 16 * batch_rq_tiles(a.q) * kp * double(tiles) / a.n_rranges);
+    return 16 * std::min<int64_t>(std::max<int64_t>(1, int64_t(s + 0.5)), tiles / 2);
+}
+
+}  // namespace
+
 int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, hipEvent_t scanned) {
     MARS_CHECK(k_out >= 1 && k_out <= batch_kpart(a.k), MARS_ERR_INVALID, "batched top-K: %d of %d kept", k_out,
                batch_kpart(a.k));
@@ -420,10 +441,12 @@ int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, 
     // K (1 + ln(rows / K)) rows per range (every new best of the rows seen so far), with
     // it about rows x K / sampled rows.
     const bool gemm = batch_uses_gemm(a.q, a.q_plain == 0);
-    if (gemm || (a.q > kRqMaxScanQ && a.rows_per_range >= kSampleDiv * kSampleRowsMin)) {
+    a.sample_pass = batch_keeps_all(a.q, a.q_plain == 0, a.rows_per_range, kp) ? 1 : 0;   // one pass, every row's key
+    const int64_t rq_rows = batch_uses_rq(a.q, a.q_plain == 0) ? rq_sample_rows(a, kp) : 0;
+    if (gemm || rq_rows > 0) {
         BatchArgs b = a;
         b.rows_per_range = gemm ? std::min<int64_t>(a.rows_per_range, (kMmSampleTiles + a.n_rranges - 1) / a.n_rranges * 256)
-                                : std::min<int64_t>(kSampleRowsMax, a.rows_per_range / kSampleDiv / 16 * 16);
+                                : rq_rows;
         b.range_stride = a.rows_per_range;
         b.sample_pass = 1;
         MARS_TRY(launch_batch_scan(b, s));

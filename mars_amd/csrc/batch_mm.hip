@@ -71,14 +71,6 @@ static_assert(kMThreads / 64 * kMDma * 64 == kMR * 4, "the waves' loads cover a 
 constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 constexpr int kWaitLgkm0 = 15 | (3 << 14) | (7 << 4);
 
-// A pointer the wave holds in SGPRs (the same in every lane), so that loads take the
-// scalar-base plus 32-bit vector-offset form.
-__device__ inline const char* uniform_ptr(const char* p) {
-    const uint64_t u = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(u)), hi = __builtin_amdgcn_readfirstlane(uint32_t(u >> 32));
-    return reinterpret_cast<const char*>((uint64_t(hi) << 32) | lo);
-}
-
 // Workgroup barrier without the memory fence of __syncthreads (which waits for every
 // load in flight, the stage prefetches included): callers wait for what they need first.
 __device__ inline void lds_barrier() {

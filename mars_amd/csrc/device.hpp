@@ -24,6 +24,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 
+// A pointer the wave holds in SGPRs (the same in every lane), so that loads take the
+// scalar-base plus 32-bit vector-offset form.
+__device__ inline const char* uniform_ptr(const char* p) {
+    const uint64_t u = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(u)), hi = __builtin_amdgcn_readfirstlane(uint32_t(u >> 32));
+    return reinterpret_cast<const char*>((uint64_t(hi) << 32) | lo);
+}
+
 // Insert key x into a register list of K keys kept ascending; x < list[K-1] is
 // checked by the caller.
 template <int K>

@@ -85,9 +85,11 @@ void dfree(T*& p) {
 
 // Row ranges x query blocks of the batched scan (defined in api.hip). plain: every query
 // is a neighbour search (BatchArgs::q_plain == 0), which picks the kernel as in
-// batch_uses_gemm. max_ranges caps the row ranges (workgroups per 64-query block).
+// batch_uses_gemm. max_ranges caps the row ranges (workgroups per 64-query block). kp: the keys
+// per query and range the launch keeps (batch_kpart), or 0; with it a k_batch_rq launch of few
+// rows gets ranges of kp rows, which keep every row (batch_keeps_all).
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
-                int32_t max_ranges = 256);
+                int32_t max_ranges = 256, int32_t kp = 0);
 
 constexpr int kMaxK = 64;              // seeds per query (wave-held list), as MAX_TOP_K
 constexpr int kSortCap = 8192;         // results sorted in LDS by the finalize kernel (one band)
@@ -537,7 +539,7 @@ bool batch_dim_supported(int32_t d);
 //   Q > kRqMaxScanQ               k_batch_rq (batch_rq.hip): the queries held in registers
 //                                 (128 or 256 per workgroup, batch_rq_tiles x 16 per wave),
 //                                 16-row tiles streamed through LDS, a sampled score floor
-//                                 (Q = 256: 549 us; Q = 1024: 1.80 ms);
+//                                 (Q = 256: 485 us the whole call);
 //   neighbour searches, Q >= kGemmMinQ
 //                                 k_batch_mm: 256-query x 256-row LDS tiles, thresholds from
 //                                 the sampled floor (the k-NN builders' 1024-query chunks:
@@ -565,15 +567,19 @@ __host__ __device__ inline int32_t mm_xcd_groups(int32_t groups) {
     return xg;
 }
 int32_t mm_ranges(int32_t groups, int64_t tiles);
-// Queries (rounded up to 64) x row ranges of any launch batch_grid lays out, at most: 256 groups x
-// ranges of 256 queries.
-constexpr int64_t kMaxRangeQueries = 256 * 256;
 // The queries per launch for a build of q queries over n rows: as many as kMmMaxQ in equal
 // launches, or 8192 (32 groups, which fill the chip evenly) when that takes fewer tile steps.
 int32_t mm_chunk(int64_t q, int64_t n);
 constexpr int32_t kRqMaxScanQ = 64;
 bool batch_uses_gemm(int32_t q, bool plain);
 bool batch_uses_rq(int32_t q, bool plain);
+// A k_batch_rq launch whose ranges hold as many rows as keys: its product is written whole, a
+// key per row, and the merge selects. batch_grid lays launches out so where a workgroup would have
+// fewer than kRqFloorTiles tiles: too few to take a floor from (rq_sample_rows), and filling and
+// searching lists costs more than a longer merge (87 global queries over 5,849 rows:
+// the whole call 178 us with lists, 157 us so).
+constexpr int64_t kRqFloorTiles = 4;
+bool batch_keeps_all(int32_t q, bool plain, int64_t rows_per_range, int32_t kp);
 int batch_rq_tiles(int32_t q);   // 16-query MFMA tiles per k_batch_rq wave: 2 or 4
 int launch_batch_rq(const BatchArgs& a, hipStream_t s);
 int batch_kpart(int32_t k);  // keys per (query, row range) the scan writes
@@ -582,17 +588,10 @@ int launch_batch_scan(const BatchArgs& a, hipStream_t s);
 int launch_batch_mm(const BatchArgs& a, hipStream_t s);
 int launch_batch_merge(const uint64_t* part, int32_t n_rranges, int32_t kpart, int32_t q, int32_t k_out,
                        uint64_t* out, hipStream_t s);
-// Scoring plus the merge: out[j * k_out ..] = query j's k_out best keys over all rows. On
-// large corpora (ranges of at least kSampleDiv kSampleRowsMin rows) a first pass over the
-// first 1 / kSampleDiv of every range (kSampleRowsMin .. kSampleRowsMax rows), merged into out, gives
-// each query a floor (its k_out-th best sampled score, a lower bound of the final one), so
-// the full pass keeps only rows at or above it.
-// At 1M rows, Q = 256: 1/64 of each range (48 rows) gives a sampled pass of 45 us and a
-// full pass of 482 us, 1/32 (112 rows) 77 and 458 us, 1/16 5% slower than 1/32; below
-// kSampleRowsMin the floor is too weak to pay for its pass.
-constexpr int64_t kSampleDiv = 64;
-constexpr int64_t kSampleRowsMin = 32;
-constexpr int64_t kSampleRowsMax = 1024;
+// Scoring plus the merge: out[j * k_out ..] = query j's k_out best keys over all rows. For more
+// than kRqMaxScanQ queries (k_batch_rq, k_batch_mm) a first pass over the first rows of every
+// range keeps maxima over classes of rows, merged into out: each query's k_out-th best is a floor
+// (a lower bound of its final one), and the full pass keeps only rows at or above it.
 // k_batch_mm samples whole tiles, kMmSampleTiles of them over its ranges at least: a query then has
 // about 16 / kMmSampleTiles dots above its floor per tile, so a wave's 64 records hold those of
 // its quarter tile (about 1024 / kMmSampleTiles). Small corpora are sampled whole: at 10K rows

@@ -154,3 +154,40 @@ def test_rq_neighbour_search(rng):
             for j in set(got[i].tolist()) ^ set(want[100 + i].tolist()):
                 assert abs(s[i, j] - sims[100 + i, 7]) <= 1e-3, (i, j)
     assert np.all(got != np.arange(100, 400)[:, None])
+
+
+# up to 3 tiles per workgroup every row's key is kept (10 to 12,289 rows: one workgroup to three
+# tiles for each of 256); from 4 on a floor and lists
+@pytest.mark.parametrize("n", [10, 41, 4097, 12_288, 12_289, 64 * 256 - 15, 64 * 256 + 1, 40_000])
+@pytest.mark.parametrize("q,k,lam,uniform", [(70, 8, LAM, False), (130, 16, LAM, True), (256, 9, 0.0, False),
+                                             (100, 16, -1e-3, False)])
+def test_rq_floors_and_queues_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng):
+    """Rows that improve along every range (the sampled first tiles give weak floors, so tiles
+    go through the dense way, the queues and their drains in turn), 40 copies of one row (ties
+    across ranges), rows of zeros and one NaN row: ids and score bits equal k_batch_scan's."""
+    d = 256
+    emb = rng.standard_normal((n, d)).astype(np.float32)
+    emb /= np.linalg.norm(emb, axis=1, keepdims=True)
+    base = emb[:8].mean(axis=0)
+    emb += (np.linspace(0.0, 3.0, n, dtype=np.float32) % 0.4)[:, None] * base
+    emb[rng.choice(n, min(n // 3, 40), replace=False)] = emb[n // 2]
+    emb[n - 5:n - 2] = 0.0
+    emb[n // 3, 7] = np.nan
+    mods = rng.integers(0, 3, size=n).astype(np.int32)
+    ts = rng.uniform(0, 600, size=n).astype(np.float32)
+    dev = Dev(emb, mods, ts, None, None, fp16=True)
+    pick = rng.choice(n, q, replace=n < q)
+    pick[pick == n // 3] = 0
+    qs = np.ascontiguousarray(emb[pick])
+    tq = np.full(q, T_Q, np.float32) if uniform else rng.uniform(300, 600, q).astype(np.float32)
+    cfg = RetrievalConfig(top_k=k, time_decay_lambda=lam, modality_filter=-1 if n % 2 else 1)
+    buf = mars_amd.DeviceBuffer.from_array(qs)
+    try:
+        ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # k_batch_rq
+        parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, min(32, q - j), tq[j:j + 32], cfg)
+                 for j in range(0, q, 32)]                                                   # k_batch_scan
+    finally:
+        buf.free()
+        dev.close()
+    np.testing.assert_array_equal(ids, np.concatenate([p[0] for p in parts]))
+    np.testing.assert_array_equal(sc.view(np.uint32), np.concatenate([p[1] for p in parts]).view(np.uint32))
