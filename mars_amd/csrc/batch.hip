@@ -13,7 +13,7 @@
 //                id asc). Workgroup (row range r, query block b) writes K keys per
 //                query; the workgroup index puts all query blocks of a row range
 //                on the same XCD (id % 8 == r % 8) so they share its L2.
-//  k_batch_merge One wave per query merges the per-row-range keys.
+//  k_batch_merge One workgroup (or wave) per query merges the per-row-range keys.
 //  k_knn_rerank  Exact fp32 rescoring of k-NN candidates (one wave per node).
 //
 //  Reference analogue: wmma_mma_similarity_kernel / wmma_similarity_kernel
@@ -223,13 +223,16 @@ __global__ __launch_bounds__(kBWaves * 64) void k_batch_scan(BatchArgs a) {
     }
 }
 
-// Merge n_rranges lists of K keys per query into the best k_out, W waves per query. Each wave
-// takes every W-th round of 8 x 64 keys (loads in flight together; a chunk with many keys
-// under the wave's bound is sorted and merged in registers, one with a few inserts them one
-// by one), then the query's first wave merges the W lists. W = 8, a workgroup per query, for
-// many ranges (256 queries of 4,096 keys: 13 us; one wave per query, every key under its bound
-// inserted one at a time: 21 us). W = 1, four queries per workgroup, where one round holds
-// all of a query's keys: the other seven waves would have none.
+// Merge n_rranges lists of K keys (in any order) per query into the best k_out, W waves per query.
+// The keys are dealt into 64 columns (lane l of every chunk; a list's keys are rotated from chunk
+// to chunk, so that ascending lists don't put their first keys into a few columns). The k_out-th
+// least of the columns' least keys is the cut: k_out keys are at or below it, so the result is
+// among those, about 18 of random keys for k_out = 16; they are gathered in LDS and sorted once.
+// (More than 64: each wave offers its keys to a list of its own, and the first merges them.)
+// (Sorting and merging every 64 keys, 27 exchange steps on 64-bit keys each time, bounded this by
+// issue: 256 queries of 4,096 keys 13.4 us, 4.7 us where all keys are empty; with the cut
+// 6.0 us.) W = 8, a workgroup per query, for many ranges. W = 1, four queries per workgroup,
+// where one round of 8 x 64 keys holds all of a query's keys: the other seven waves would have none.
 constexpr int kMergeWaves = 8;
 constexpr int kMergeLd = 8;
 constexpr int kRerankPieces = 3;  // k_knn_rerank: 16-byte pieces per lane and row (d <= 768)
@@ -237,37 +240,103 @@ template <int W>
 __global__ __launch_bounds__(W == 1 ? 256 : W * 64) void k_batch_merge(const uint64_t* __restrict__ part,
                                                                       int32_t n_rranges, int32_t kpart, int32_t q,
                                                                       int32_t k_out, uint64_t* __restrict__ out) {
-    __shared__ uint64_t s_l[W][64];
+    __shared__ uint64_t s_l[W == 1 ? 4 : W][64];
+    __shared__ uint64_t s_best[W == 1 ? 4 : 1][64];
+    __shared__ uint32_t s_n;
     const int lane = int(threadIdx.x & 63u), w0 = int(threadIdx.x >> 6);
     const int wave = W == 1 ? 0 : w0;                  // of the query's W
     const int qi = W == 1 ? int(blockIdx.x) * 4 + w0 : int(blockIdx.x);
     if (qi >= q) return;                               // the whole workgroup, or (W = 1) the wave
     const int qb = qi / kBQ, j = qi % kBQ;
-    uint64_t list = kEmptyKey, thr = kEmptyKey;
     const int total = n_rranges * kpart;
     const int kshift = kpart == 8 ? 3 : 4;             // kpart is 8 or 16 (batch_kpart)
-    for (int base = wave * 64 * kMergeLd; base < total; base += W * 64 * kMergeLd) {
-        uint64_t xs[kMergeLd];
+    const auto load = [&](int base, uint64_t (&xs)[kMergeLd]) {
 #pragma unroll
         for (int c = 0; c < kMergeLd; ++c) {
             const int t = base + c * 64 + lane;
-            xs[c] = kEmptyKey;
-            if (t < total) {
-                const int r = t >> kshift, s = t & (kpart - 1);
-                xs[c] = part[((int64_t(qb) * n_rranges + r) * kBQ + j) * kpart + s];
-            }
+            const bool on = t < total;                 // (total is a multiple of kpart: whole lists)
+            const int list = on ? t >> kshift : 0;
+            const uint64_t x =
+                part[((int64_t(qb) * n_rranges + list) * kBQ + j) * kpart + ((t + (t >> 6)) & (kpart - 1))];
+            xs[c] = on ? x : kEmptyKey;
         }
+    };
+    // the first round's keys stay in registers; later rounds' (many ranges) are read again
+    const int first = wave * 64 * kMergeLd, step = W * 64 * kMergeLd;
+    uint64_t xs[kMergeLd], least = kEmptyKey;
+    load(first, xs);
 #pragma unroll
-        for (int c = 0; c < kMergeLd; ++c) wave_offer(list, thr, xs[c], lane, k_out);
+    for (int c = 0; c < kMergeLd; ++c) least = xs[c] < least ? xs[c] : least;
+    for (int base = first + step; base < total; base += step) {
+        uint64_t ys[kMergeLd];
+        load(base, ys);
+#pragma unroll
+        for (int c = 0; c < kMergeLd; ++c) least = ys[c] < least ? ys[c] : least;
     }
     if constexpr (W > 1) {
-        s_l[wave][lane] = list;
+        s_l[wave][lane] = least;
+        if (threadIdx.x == 0) s_n = 0u;
         __syncthreads();
-        if (wave != 0) return;
 #pragma unroll
-        for (int w = 1; w < W; ++w) list = wave_merge64(list, s_l[w][lane], lane, k_out);
+        for (int w = 0; w < W; ++w) least = s_l[w][lane] < least ? s_l[w][lane] : least;
     }
-    if (lane < k_out) out[int64_t(qi) * k_out + lane] = list;
+    const uint64_t cut = __shfl(wave_sort64(least, lane), k_out - 1);
+    // the keys at or below the cut, gathered
+    uint64_t* const best = s_best[W == 1 ? w0 : 0];
+    uint32_t n = 0;                                    // W = 1: gathered so far
+    const auto gather = [&](const uint64_t (&x)[kMergeLd]) {
+        uint32_t mine = 0, at = 0;
+#pragma unroll
+        for (int c = 0; c < kMergeLd; ++c) mine += uint32_t(__popcll(__ballot(x[c] <= cut && x[c] != kEmptyKey)));
+        if (mine == 0) return;
+        if constexpr (W == 1) {
+            at = n;
+            n += mine;
+        } else {
+            if (lane == 0) at = atomicAdd(&s_n, mine);
+            at = __builtin_amdgcn_readfirstlane(at);
+        }
+#pragma unroll
+        for (int c = 0; c < kMergeLd; ++c) {
+            const bool on = x[c] <= cut && x[c] != kEmptyKey;
+            const uint64_t b = __ballot(on);
+            const uint32_t i = at + __builtin_amdgcn_mbcnt_hi(uint32_t(b >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(b), 0u));
+            if (on && i < 64u) best[i] = x[c];
+            at += uint32_t(__popcll(b));
+        }
+    };
+    gather(xs);
+    for (int base = first + step; base < total; base += step) {
+        uint64_t ys[kMergeLd];
+        load(base, ys);
+        gather(ys);
+    }
+    if constexpr (W > 1) {
+        __syncthreads();
+        n = s_n;
+    }
+    uint64_t list = kEmptyKey;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (n <= 64u) {                                    // uniform over the query's waves
+        if (wave == 0) list = wave_sort64(uint32_t(lane) < n ? best[lane] : kEmptyKey, lane);
+    } else {
+        uint64_t thr = kEmptyKey;
+#pragma unroll
+        for (int c = 0; c < kMergeLd; ++c) wave_offer(list, thr, xs[c] <= cut ? xs[c] : kEmptyKey, lane, k_out);
+        for (int base = first + step; base < total; base += step) {
+            load(base, xs);
+#pragma unroll
+            for (int c = 0; c < kMergeLd; ++c) wave_offer(list, thr, xs[c] <= cut ? xs[c] : kEmptyKey, lane, k_out);
+        }
+        if constexpr (W > 1) {
+            s_l[wave][lane] = list;
+            __syncthreads();
+            if (wave == 0)
+                for (int w = 1; w < W; ++w) list = wave_merge64(list, s_l[w][lane], lane, k_out);
+        }
+    }
+    if (wave == 0 && lane < k_out) out[int64_t(qi) * k_out + lane] = list;
 }
 
 // Exact fp32 rescoring of kc candidates per node; keeps k_out by (score desc, id asc).

@@ -191,3 +191,28 @@ def test_rq_floors_and_queues_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng)
         dev.close()
     np.testing.assert_array_equal(ids, np.concatenate([p[0] for p in parts]))
     np.testing.assert_array_equal(sc.view(np.uint32), np.concatenate([p[1] for p in parts]).view(np.uint32))
+
+
+# one merge wave's 512 keys (32 ranges of 16, 64 of 8), more lists, ragged ones
+@pytest.mark.parametrize("n", [5, 500, 512, 520, 1040, 4096, 9000])
+@pytest.mark.parametrize("q,k", [(1, 1), (33, 8), (64, 16), (3, 9)])
+def test_merge_of_few_and_many_keys(n, q, k, rng):
+    """k_batch_merge on lists with equal keys' scores (60 copies of one row), whose cut lets more
+    than 64 keys through, and on fewer keys than asked for: the oracle's top-K by (score, id)."""
+    d = 256
+    emb, mods, ts, _, _, _ = random_graph(rng, n, d)
+    emb[: min(n, 60)] = emb[0]
+    ts[:] = 0.0
+    dev = Dev(emb, mods, ts, None, None, fp16=True)
+    buf = mars_amd.DeviceBuffer.from_array(np.ascontiguousarray(np.repeat(emb[:1], q, axis=0)))
+    try:
+        ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, np.zeros(q, np.float32),
+                                       RetrievalConfig(top_k=k, time_decay_lambda=0.0))
+    finally:
+        buf.free()
+        dev.close()
+    want = np.full(k, -1)
+    want[: min(n, k)] = np.arange(min(n, k))                 # the copies, least ids first
+    np.testing.assert_array_equal(ids, np.tile(want, (q, 1)))
+    live = want >= 0
+    assert np.all(sc[:, live] == sc[0, 0]) and abs(sc[0, 0] - 1.0) < 2e-3
