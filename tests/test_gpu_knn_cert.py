@@ -165,3 +165,29 @@ def test_build_grids(n, first, count):
         check_lists(c.embeddings, first + idx, got[idx])
     finally:
         mars_amd.free_device(dg)
+
+
+@pytest.mark.parametrize("k", [1, 3, 4, 8, 15, 16])
+def test_rescoring_that_stops_early_is_exact(k):
+    """Rows spaced so that fp16 scores order some candidates wrongly (copies with perturbations
+    near the fp16 step) among well separated ones: every list equals the oracle's, whether the
+    rescoring ran through all 16 candidates or stopped after the first k."""
+    c = corpus.make_corpus(2100, 512, seed=23)
+    emb = c.embeddings.copy()
+    rng = np.random.default_rng(24)
+    for base in range(0, 2000, 50):
+        e = emb[base] + rng.uniform(0, 6e-4, (20, 1)).astype(np.float32) * rng.standard_normal((20, 512)).astype(np.float32)
+        emb[base + 1:base + 21] = e / np.linalg.norm(e, axis=1, keepdims=True)
+    dg = device_graph(emb, c.modalities, c.timestamps)
+    try:
+        got = mars_amd.graph_knn(dg, k)
+        u, r = dg.knn_report
+        assert r == u
+    finally:
+        mars_amd.free_device(dg)
+    s = emb.astype(np.float64) @ emb.astype(np.float64).T
+    np.fill_diagonal(s, -np.inf)
+    kth = np.sort(s, axis=1)[:, -k]
+    took = np.take_along_axis(s, got, axis=1)
+    assert np.all(took >= kth[:, None] - 1e-6)              # fp32 sums of 512 products of unit rows
+    assert all(len(set(row)) == k for row in got.tolist())
