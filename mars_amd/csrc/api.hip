@@ -1958,6 +1958,112 @@ int knn_rescan_uncertified(mars_graph* gh, int32_t k, int64_t first, const std::
     return rc;
 }
 
+// What a builder call needs on the device, in one allocation kept by the graph (under its mutex; up
+// to kKnnKeep bytes, larger ones are freed after the call) with the stream: five allocations, their
+// release and a stream per call took 100 us, a fifth of the 8-NN graph of 10K rows.
+constexpr size_t kKnnKeep = size_t(64) << 20;
+constexpr size_t kKnnPinned = size_t(4) << 20;       // staging of results (larger ones are copied directly)
+int knn_workspace(Graph& g, size_t bytes, size_t results) {
+    if (!g.knn_stream) MARS_HIP(hipStreamCreateWithFlags(&g.knn_stream, hipStreamNonBlocking));
+    if (bytes > g.knn_ws_bytes) {
+        if (g.knn_ws) (void)hipFree(g.knn_ws);
+        g.knn_ws = nullptr;
+        g.knn_ws_bytes = 0;
+        unsigned char* p = nullptr;
+        MARS_TRY(dmalloc(&p, bytes));
+        g.knn_ws = p;
+        g.knn_ws_bytes = bytes;
+    }
+    if (results <= kKnnPinned && results > g.knn_pin_bytes) {
+        if (g.knn_pin) (void)hipHostFree(g.knn_pin);
+        g.knn_pin = nullptr;
+        g.knn_pin_bytes = 0;
+        if (hipHostMalloc(&g.knn_pin, results, hipHostMallocDefault) == hipSuccess) g.knn_pin_bytes = results;
+        else {
+            g.knn_pin = nullptr;                     // copied directly
+            (void)hipGetLastError();
+        }
+    }
+    return MARS_OK;
+}
+
+// The k-NN lists of nodes [lo, hi), certified (cert[i]: node lo + i's list is exact), ids as
+// searched: block > 0: each node among its own block of that many rows (relative to the block's
+// first; lo is one), block = 0: among all rows.
+int knn_lists(Graph& g, int32_t k, int64_t lo, int64_t hi, int64_t block, int32_t* nbrs, std::vector<int32_t>& hcert) {
+    constexpr int32_t kCand = 16;
+    const int64_t n = g.n, count = hi - lo, most = block ? std::min(block, count) : count;
+    const int32_t chunk = mm_chunk(block ? block : count, block ? block : n);   // queries per launch
+    int32_t nrr = 0, nqb = 0;
+    int64_t rpr = 0;
+    int64_t part_keys = 0;                           // the largest launch's
+    for (const int64_t nb : {most, block ? count % block : 0}) {
+        for (const int64_t q : {std::min<int64_t>(chunk, nb), nb % chunk}) {
+            if (q == 0) continue;
+            batch_grid(block ? nb : n, int32_t(q), true, &nrr, &nqb, &rpr, 256, kCand);
+            part_keys = std::max(part_keys, int64_t(nqb) * nrr * 64 * kCand);
+        }
+    }
+    const auto pad = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t n_dn = size_t(count) * k * sizeof(int32_t), n_cert = size_t(count) * sizeof(int32_t);
+    const size_t o_dn = 0, o_cert = pad(n_dn), o_tq = o_cert + pad(n_cert), o_cand = o_tq + pad(size_t(chunk) * sizeof(float)),
+                 o_part = o_cand + pad(size_t(chunk) * kCand * sizeof(uint64_t)),
+                 bytes = o_part + size_t(part_keys) * sizeof(uint64_t);
+    MARS_TRY(knn_workspace(g, bytes, o_cert + n_cert));
+    unsigned char* const ws = static_cast<unsigned char*>(g.knn_ws);
+    int32_t* const dn = reinterpret_cast<int32_t*>(ws + o_dn);
+    int32_t* const cert = reinterpret_cast<int32_t*>(ws + o_cert);
+    float* const tq = reinterpret_cast<float*>(ws + o_tq);
+    uint64_t* const cand = reinterpret_cast<uint64_t*>(ws + o_cand);
+    uint64_t* const part = reinterpret_cast<uint64_t*>(ws + o_part);
+    hipStream_t s = g.knn_stream;
+    int rc = MARS_OK;
+    hipError_t e = hipMemsetAsync(tq, 0, size_t(chunk) * sizeof(float), s);
+    if (e == hipSuccess && !g.nrm) e = hipMemsetAsync(cert, 0, n_cert, s);
+    // rows [r0, r0 + rows), queries [q0, q1): rows, queries and candidate ids relative to r0
+    for (int64_t b0 = lo; b0 < hi && rc == MARS_OK && e == hipSuccess; b0 += block ? block : count) {
+        const int64_t r0 = block ? b0 : 0, rows = block ? std::min(block, n - b0) : n, q1 = block ? b0 + rows : hi;
+        for (int64_t q0 = b0; q0 < q1 && rc == MARS_OK; q0 += chunk) {
+            const int32_t q = int32_t(std::min<int64_t>(chunk, q1 - q0));
+            batch_grid(rows, q, true, &nrr, &nqb, &rpr, 256, kCand);
+            BatchArgs a{};
+            a.emb16 = g.emb16 + r0 * g.d; a.n = rows; a.d = g.d; a.qh = g.emb16 + q0 * g.d; a.q = q; a.tq = tq;
+            a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm;
+            a.q_plain = 0; a.self_base = q0 - r0; a.part = part; a.uniform_tq = 1;
+            a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
+            rc = launch_batch_topk(a, kCand, cand, s);
+            if (rc == MARS_OK)
+                rc = launch_knn_rerank(g.emb + r0 * g.d, q0 - r0, q, g.d, cand, kCand, k, dn + (q0 - lo) * k, s, g.nrm,
+                                       g.nrm ? cert + (q0 - lo) : nullptr);
+        }
+    }
+    hcert.assign(size_t(count), 0);
+    const size_t results = o_cert + n_cert;
+    if (rc == MARS_OK && e == hipSuccess) {
+        if (results <= g.knn_pin_bytes) {
+            e = hipMemcpyAsync(g.knn_pin, ws, results, hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipStreamSynchronize(s);
+            if (e == hipSuccess) {
+                std::memcpy(nbrs, g.knn_pin, n_dn);
+                std::memcpy(hcert.data(), static_cast<unsigned char*>(g.knn_pin) + o_cert, n_cert);
+            }
+        } else {
+            e = hipStreamSynchronize(s);
+            if (e == hipSuccess) e = hipMemcpy(nbrs, dn, n_dn, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(hcert.data(), cert, n_cert, hipMemcpyDeviceToHost);
+        }
+    } else {
+        (void)hipStreamSynchronize(s);               // nothing may use the workspace after the call
+    }
+    if (rc == MARS_OK && e != hipSuccess) rc = set_error(MARS_ERR_HIP, "k-NN: %s", hipGetErrorString(e));
+    if (g.knn_ws_bytes > kKnnKeep) {
+        (void)hipFree(g.knn_ws);
+        g.knn_ws = nullptr;
+        g.knn_ws_bytes = 0;
+    }
+    return rc;
+}
+
 }  // namespace
 
 int mars_graph_knn_report(const mars_graph* gh, int64_t* uncertified, int64_t* rescanned) {
@@ -1983,66 +2089,13 @@ int mars_graph_knn_blocks(mars_graph* gh, int32_t k, int32_t block_rows, int32_t
     MARS_CHECK(g.emb16 != nullptr, MARS_ERR_UNSUPPORTED, "k-NN reads the fp16 corpus: enable it first");
     MARS_CHECK(batch_dim_supported(g.d), MARS_ERR_UNSUPPORTED, "k-NN: embedding_dim %d unsupported", g.d);
     MARS_TRY(use_device(g.device));
-    constexpr int32_t kCand = 16;
     const int64_t B = std::min<int64_t>(block_rows, g.n);
-    const int32_t chunk = mm_chunk(B, B);            // queries per launch
     // nodes [lo, hi): the requested blocks
     const int64_t lo = std::min<int64_t>(int64_t(first_block) * block_rows, g.n);
     const int64_t hi = std::min<int64_t>(lo + int64_t(n_blocks) * block_rows, g.n);
     if (hi <= lo) return MARS_OK;
-    int32_t nrr = 0, nqb = 0;
-    int64_t rpr = 0;
-    int64_t part_keys = 0;                           // the largest launch's
-    for (const int64_t nb : {B, (hi - lo) % B}) {
-        for (const int64_t q : {std::min<int64_t>(chunk, nb), nb % chunk}) {
-            if (q == 0) continue;
-            batch_grid(nb, int32_t(q), true, &nrr, &nqb, &rpr, 256, kCand);
-            part_keys = std::max(part_keys, int64_t(nqb) * nrr * 64 * kCand);
-        }
-    }
-    float* tq = nullptr; uint64_t* part = nullptr; uint64_t* cand = nullptr; int32_t* dn = nullptr;
-    int32_t* cert = nullptr;
-    hipStream_t s = nullptr;
-    int rc = MARS_OK;
-    auto cleanup = [&]() {
-        dfree(tq); dfree(part); dfree(cand); dfree(dn); dfree(cert);
-        if (s) (void)hipStreamDestroy(s);
-    };
-    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(part_keys))) ||
-        (rc = dmalloc(&cand, size_t(chunk) * kCand)) || (rc = dmalloc(&dn, size_t(hi - lo) * k)) ||
-        (rc = dmalloc(&cert, size_t(hi - lo)))) {
-        cleanup();
-        return rc;
-    }
-    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMemsetAsync(tq, 0, size_t(chunk) * sizeof(float), s);
-    if (e == hipSuccess) e = hipMemsetAsync(cert, 0, size_t(hi - lo) * sizeof(int32_t), s);
-    if (e != hipSuccess) { cleanup(); return set_error(MARS_ERR_HIP, "k-NN setup: %s", hipGetErrorString(e)); }
-    // block [r0, r1): rows, queries and candidate ids relative to r0
-    for (int64_t r0 = lo; r0 < hi && rc == MARS_OK; r0 += B) {
-        const int64_t nb = std::min<int64_t>(B, g.n - r0);
-        for (int64_t q0 = 0; q0 < nb && rc == MARS_OK; q0 += chunk) {
-            const int32_t q = int32_t(std::min<int64_t>(chunk, nb - q0));
-            batch_grid(nb, q, true, &nrr, &nqb, &rpr, 256, kCand);
-            BatchArgs a{};
-            a.emb16 = g.emb16 + r0 * g.d; a.n = nb; a.d = g.d; a.qh = g.emb16 + (r0 + q0) * g.d; a.q = q; a.tq = tq;
-            a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
-            a.part = part; a.uniform_tq = 1;
-            a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
-            rc = launch_batch_topk(a, kCand, cand, s);
-            if (rc == MARS_OK)
-                rc = launch_knn_rerank(g.emb + r0 * g.d, q0, q, g.d, cand, kCand, k, dn + (r0 - lo + q0) * k, s,
-                                       g.nrm, g.nrm ? cert + (r0 - lo + q0) : nullptr);
-        }
-    }
-    std::vector<int32_t> hcert(size_t(hi - lo), 0);
-    if (rc == MARS_OK) {
-        e = hipStreamSynchronize(s);
-        if (e == hipSuccess) e = hipMemcpy(nbrs, dn, size_t(hi - lo) * k * sizeof(int32_t), hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(hcert.data(), cert, hcert.size() * sizeof(int32_t), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) rc = set_error(MARS_ERR_HIP, "k-NN: %s", hipGetErrorString(e));
-    }
-    cleanup();
+    std::vector<int32_t> hcert;
+    int rc = knn_lists(g, k, lo, hi, B, nbrs, hcert);
     if (rc == MARS_OK && B < g.n) {                      // block-relative ids -> node ids
         for (int64_t i = lo; i < hi; ++i) {
             const int32_t off = int32_t(i / B * B);
@@ -2067,57 +2120,9 @@ int mars_graph_knn_range(mars_graph* gh, int32_t k, int32_t first, int32_t count
                (long long)first + count, g.n);
     if (count == 0) return MARS_OK;
     MARS_TRY(use_device(g.device));
-    constexpr int32_t kCand = 16;
-    const int64_t n = g.n;
-    const int32_t chunk = mm_chunk(count, n);        // queries per launch
-    int32_t nrr = 0, nqb = 0;
-    int64_t rpr = 0;
-    int64_t part_keys = 0;                           // the largest launch's
-    for (const int64_t q : {std::min<int64_t>(chunk, count), int64_t(count % chunk)}) {
-        if (q == 0) continue;
-        batch_grid(n, int32_t(q), true, &nrr, &nqb, &rpr, 256, kCand);
-        part_keys = std::max(part_keys, int64_t(nqb) * nrr * 64 * kCand);
-    }
-    float* tq = nullptr; uint64_t* part = nullptr; uint64_t* cand = nullptr; int32_t* dn = nullptr;
-    int32_t* cert = nullptr;
-    hipStream_t s = nullptr;
-    int rc = MARS_OK;
-    auto cleanup = [&]() {
-        dfree(tq); dfree(part); dfree(cand); dfree(dn); dfree(cert);
-        if (s) (void)hipStreamDestroy(s);
-    };
-    if ((rc = dmalloc(&tq, size_t(chunk))) || (rc = dmalloc(&part, size_t(part_keys))) ||
-        (rc = dmalloc(&cand, size_t(chunk) * kCand)) || (rc = dmalloc(&dn, size_t(count) * k)) ||
-        (rc = dmalloc(&cert, size_t(count)))) {
-        cleanup();
-        return rc;
-    }
-    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMemsetAsync(tq, 0, size_t(chunk) * sizeof(float), s);
-    if (e == hipSuccess) e = hipMemsetAsync(cert, 0, size_t(count) * sizeof(int32_t), s);
-    if (e != hipSuccess) { cleanup(); return set_error(MARS_ERR_HIP, "k-NN range setup: %s", hipGetErrorString(e)); }
-    // queries [q0, q0 + q) against every node; the query's own id is excluded
-    for (int64_t q0 = first; q0 < int64_t(first) + count && rc == MARS_OK; q0 += chunk) {
-        const int32_t q = int32_t(std::min<int64_t>(chunk, int64_t(first) + count - q0));
-        batch_grid(n, q, true, &nrr, &nqb, &rpr, 256, kCand);
-        BatchArgs a{};
-        a.emb16 = g.emb16; a.n = n; a.d = g.d; a.qh = g.emb16 + q0 * g.d; a.q = q; a.tq = tq;
-        a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm; a.q_plain = 0; a.self_base = q0;
-        a.part = part; a.uniform_tq = 1;
-        a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
-        rc = launch_batch_topk(a, kCand, cand, s);
-        if (rc == MARS_OK)
-            rc = launch_knn_rerank(g.emb, q0, q, g.d, cand, kCand, k, dn + (q0 - first) * k, s, g.nrm,
-                                   g.nrm ? cert + (q0 - first) : nullptr);
-    }
-    std::vector<int32_t> hcert(static_cast<size_t>(count), 0);
-    if (rc == MARS_OK) {
-        e = hipStreamSynchronize(s);
-        if (e == hipSuccess) e = hipMemcpy(nbrs, dn, size_t(count) * k * sizeof(int32_t), hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(hcert.data(), cert, hcert.size() * sizeof(int32_t), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) rc = set_error(MARS_ERR_HIP, "k-NN range: %s", hipGetErrorString(e));
-    }
-    cleanup();
+    // the nodes against every node; a node's own id is excluded
+    std::vector<int32_t> hcert;
+    int rc = knn_lists(g, k, first, int64_t(first) + count, 0, nbrs, hcert);
     if (rc == MARS_OK) rc = knn_rescan_uncertified(gh, k, first, hcert, nbrs, true);
     return rc;
 }

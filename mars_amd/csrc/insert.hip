@@ -560,6 +560,12 @@ int graph_insert_free(Graph& g) {
     dfree(g.ins8_part); dfree(g.ins8_qa); dfree(g.ins8_qp); dfree(g.ins8_stat); dfree(g.ins8_margin); dfree(g.ins_cert);
     g.ins_part_cap = 0;
     g.ins_cap_q = 0;
+    if (g.knn_ws) (void)hipFree(g.knn_ws);
+    if (g.knn_pin) (void)hipHostFree(g.knn_pin);
+    if (g.knn_stream) (void)hipStreamDestroy(g.knn_stream);
+    g.knn_ws = g.knn_pin = nullptr;
+    g.knn_ws_bytes = g.knn_pin_bytes = 0;
+    g.knn_stream = nullptr;
     for (auto& e : g.ins_ev) {
         if (e) (void)hipEventDestroy(e);
         e = nullptr;

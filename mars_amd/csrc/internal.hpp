@@ -177,6 +177,12 @@ struct Graph {
     float* ins_tq = nullptr;             // zero query times (no decay)
     int32_t ins_cap_q = 0;
     hipEvent_t ins_ev[2] = {nullptr, nullptr};
+    // the k-NN builders' scratch (under the graph mutex): device, pinned results, stream
+    void* knn_ws = nullptr;
+    size_t knn_ws_bytes = 0;
+    void* knn_pin = nullptr;
+    size_t knn_pin_bytes = 0;
+    hipStream_t knn_stream = nullptr;
     // the last k-NN builder call: nodes whose lists the certificate did not cover, and of
     // those, how many were found again by exact scans
     int64_t knn_uncertified = 0;
