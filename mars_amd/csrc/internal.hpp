@@ -581,10 +581,11 @@ bool batch_uses_gemm(int32_t q, bool plain);
 bool batch_uses_rq(int32_t q, bool plain);
 // A k_batch_rq launch whose ranges hold as many rows as keys: its product is written whole, a
 // key per row, and the merge selects. batch_grid lays launches out so where a workgroup would have
-// fewer than kRqFloorTiles tiles: too few to take a floor from (rq_sample_rows), and filling and
-// searching lists costs more than a longer merge (87 global queries over 5,849 rows:
-// the whole call 178 us with lists, 157 us so).
-constexpr int64_t kRqFloorTiles = 4;
+// fewer than kRqFloorTiles tiles: there a floor's passes (rq_sample_rows) and filling and searching
+// lists cost more than a longer merge. (The whole call, with lists and floor / so: 438 queries
+// over 6,307 rows, 4 tiles, 90 / 74 us; 512 over 12,000, 6 tiles, 117 / 90; 256 over 40,000, 10
+// tiles, 122 / 110; 100 over 50,000, 13 tiles, 98 / 98; 80 over 60,000, 15 tiles, 88 / 106 us.)
+constexpr int64_t kRqFloorTiles = 12;
 bool batch_keeps_all(int32_t q, bool plain, int64_t rows_per_range, int32_t kp);
 int batch_rq_tiles(int32_t q);   // 16-query MFMA tiles per k_batch_rq wave: 2 or 4
 int launch_batch_rq(const BatchArgs& a, hipStream_t s);

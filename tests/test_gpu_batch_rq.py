@@ -156,9 +156,9 @@ def test_rq_neighbour_search(rng):
     assert np.all(got != np.arange(100, 400)[:, None])
 
 
-# up to 3 tiles per workgroup every row's key is kept (10 to 12,289 rows: one workgroup to three
-# tiles for each of 256); from 4 on a floor and lists
-@pytest.mark.parametrize("n", [10, 41, 4097, 12_288, 12_289, 64 * 256 - 15, 64 * 256 + 1, 40_000])
+# below 12 tiles for each of 256 workgroups every row's key is kept (10 rows to 45,056); from there
+# on a floor and lists
+@pytest.mark.parametrize("n", [10, 41, 4097, 12_289, 11 * 4096, 11 * 4096 + 1, 50_000])
 @pytest.mark.parametrize("q,k,lam,uniform", [(70, 8, LAM, False), (130, 16, LAM, True), (256, 9, 0.0, False),
                                              (100, 16, -1e-3, False)])
 def test_rq_floors_and_queues_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng):
