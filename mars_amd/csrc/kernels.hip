@@ -172,6 +172,7 @@ struct FinShared {
     int32_t seed_id[64];                 // the seeds' node ids (visit positions 0 .. ns - 1)
     int s_wave[kFinWaves];
     int s_misc[8];
+    uint64_t bound;                      // no key above it is among the rk best of the BFS (bfs_lds)
 };
 
 __device__ inline uint32_t hash_slot0(int32_t v) { return (uint32_t(v) * 2654435761u) >> (32 - 13); }
@@ -276,6 +277,10 @@ __device__ inline int round_rank(FinShared& sh, bool won, int* rank) {
 // with error <= a.eps per fused score, and writes a bound on each node's error to
 // a.vdv; `best` then tracks lower ends (score - bound, rounded down). A non-finite
 // score or bound sets sh.s_misc[7].
+// The waves share a bound on the rk-th best key (sh.bound, the least of their rk-th keys; the
+// seeds' from the start where there are rk of them): keys above it are not offered. Sorting and
+// merging every wave's 64 emitted keys per round of 1024 edges took 2-3 us of the BFS: k = 32
+// seeds, 32 results, 4,436 nodes 36.5 -> 34.8 us; interval mode, 1,184 nodes 18.7 -> 16.1 us.
 constexpr int kBfsUnscored = 0, kBfsScored = 1, kBfsInterval = 2;
 template <int MODE>
 __device__ int bfs_lds(FinShared& sh, const FinalizeArgs& a, int ns, int* levels_out, uint64_t& best,
@@ -283,7 +288,7 @@ __device__ int bfs_lds(FinShared& sh, const FinalizeArgs& a, int ns, int* levels
     constexpr int R = 4;                       // 1024-edge rounds cached in registers
     const int tid = int(threadIdx.x);
     for (int i = tid; i < kHashCap; i += kFinThreads) { sh.u.bfs.hkey[i] = 0u; sh.u.bfs.hval[i] = 0xFFFFFFFFu; }
-    if (tid == 0) { sh.s_misc[4] = 0; sh.s_misc[5] = 0; }
+    if (tid == 0) { sh.s_misc[4] = 0; sh.s_misc[5] = 0; sh.bound = bthr; }   // wave 0's: the seeds' rk-th
     __syncthreads();
     if (tid < ns) {
         const int slot = hash_find_or_insert(sh, sh.seed_id[tid]);
@@ -367,9 +372,13 @@ __device__ int bfs_lds(FinShared& sh, const FinalizeArgs& a, int ns, int* levels
                         if (pos < kRoCache) sh.ro_cache[pos] = rw[r];
                         sh.u.bfs.hval[slot[r]] = (uint32_t(h + 1) << 16) | uint32_t(pos);
                     }
-                    if (MODE == kBfsScored && rk > 0)
-                        wave_offer(best, bthr, won ? make_key(sc, uint32_t(nb[r])) : kEmptyKey, lane_id(), rk);
-                    if (MODE == kBfsInterval && rk > 0) wave_offer(best, bthr, lkey, lane_id(), rk);
+                    if (MODE != kBfsUnscored && rk > 0) {
+                        if constexpr (MODE == kBfsScored) lkey = won ? make_key(sc, uint32_t(nb[r])) : kEmptyKey;
+                        const uint64_t bound = *const_cast<volatile uint64_t*>(&sh.bound);
+                        wave_offer(best, bthr, lkey <= bound ? lkey : kEmptyKey, lane_id(), rk);
+                        if (bthr < bound && lane_id() == 0)
+                            atomicMin(reinterpret_cast<unsigned long long*>(&sh.bound), (unsigned long long)bthr);
+                    }
                     out += wtot;
                     __syncthreads();
                 }
@@ -586,26 +595,78 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(FinalizeArgs a) {
     // Every key of the K best is <= the scan's final bound (the smallest workgroup K-th
     // key), so keys above it are dropped as they load and never reach the lists.
     const uint64_t gb = *a.gthr;
-    {
-        uint64_t x[8];
+    // The keys in 64 columns (the lanes of all waves): k keys are <= the k-th least of the columns'
+    // least keys, so only keys at or below that cut are gathered and sorted, about k ln(64 / (64 -
+    // k)) 64 / k of them (45 at k = 32). (Sorting every 64 keys into each wave's list bounded this by
+    // issue: k = 32 of 512 workgroups' keys 24 -> 5 us.)
+    uint64_t x[8], least = kEmptyKey;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = a.part[wave * 64 + j * kFinThreads + lane];
+    for (int j = 0; j < 8; ++j) x[j] = a.part[wave * 64 + j * kFinThreads + lane];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            wave_offer(list, thr, (wave * 64 + j * kFinThreads + lane < n_part && x[j] <= gb) ? x[j] : kEmptyKey,
-                       lane, k);
+    for (int j = 0; j < 8; ++j) {
+        x[j] = wave * 64 + j * kFinThreads + lane < n_part && x[j] <= gb ? x[j] : kEmptyKey;
+        least = x[j] < least ? x[j] : least;
     }
-    for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
-        uint64_t x[8];
+    auto load_more = [&](int base, uint64_t (&y)[8]) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int i = base + j * kFinThreads + lane;
-            x[j] = (i < n_part) ? a.part[i] : kEmptyKey;
+            y[j] = i < n_part ? a.part[i] : kEmptyKey;
+            y[j] = y[j] <= gb ? y[j] : kEmptyKey;
         }
+    };
+    for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
+        uint64_t y[8];
+        load_more(base, y);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) wave_offer(list, thr, x[j] <= gb ? x[j] : kEmptyKey, lane, k);
+        for (int j = 0; j < 8; ++j) least = y[j] < least ? y[j] : least;
     }
-    list = tree_merge(sh, list, k, n_part <= kFinThreads ? (n_part + 63) / 64 : kFinWaves);
+    sh.lists[wave][lane] = least;
+    if (tid == 0) sh.s_misc[4] = 0;
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+        for (int w = 1; w < kFinWaves; ++w) least = sh.lists[w][lane] < least ? sh.lists[w][lane] : least;
+        const uint64_t kth = __shfl(wave_sort64(least, lane), k - 1);
+        if (lane == 0) sh.bound = kth;
+    }
+    __syncthreads();
+    const uint64_t cut = sh.bound;
+    uint64_t* const buf = sh.u.sort.key;                 // kSortCap keys
+    auto gather = [&](const uint64_t (&y)[8]) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (y[j] <= cut && y[j] != kEmptyKey) {
+                const int at = atomicAdd(&sh.s_misc[4], 1);
+                if (at < kFinThreads) buf[at] = y[j];
+            }
+        }
+    };
+    gather(x);
+    for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
+        uint64_t y[8];
+        load_more(base, y);
+        gather(y);
+    }
+    __syncthreads();
+    const int n_cut = sh.s_misc[4];
+    if (n_cut <= kFinThreads) {
+        if (wave * 64 < n_cut) {
+            list = wave_sort64(tid < n_cut ? buf[tid] : kEmptyKey, lane);
+            if (lane >= k) list = kEmptyKey;
+        }
+        list = tree_merge(sh, list, k, (n_cut + 63) / 64);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) wave_offer(list, thr, x[j] <= cut ? x[j] : kEmptyKey, lane, k);
+        for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
+            uint64_t y[8];
+            load_more(base, y);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) wave_offer(list, thr, y[j] <= cut ? y[j] : kEmptyKey, lane, k);
+        }
+        list = tree_merge(sh, list, k);
+    }
     if (wave == 0) {
         const int ns = __popcll(__ballot(lane < k && list != kEmptyKey));
         if (lane < ns) {
@@ -870,6 +931,14 @@ __device__ uint64_t merge_lists8(FinShared& sh, const uint64_t* part, int nl, in
 //    k-th exact score above (c-th fp16 score + that bound) makes the seeds the fp32 scan's.
 //  * int8 scan (upper = 1): the keys are per-row upper bounds of the fp32 scan's score,
 //    so a k-th exact score above the c-th candidate's key score is the certificate.
+// dot_all where its registers fit beside the query's (1024 threads have 128 each), else dot: the
+// same arithmetic.
+template <typename QF>
+__device__ inline float cert_dot(const QF& qf, const float* row, int sub) {
+    if constexpr (sizeof(QF) <= 12 * 16) return qf.dot_all(row, sub);
+    else return qf.dot(row, sub);
+}
+
 template <typename QF>
 __global__ __launch_bounds__(kFinThreads) void k_cert_bfs(CertArgs a, MultiArgs m) {
     __shared__ FinShared sh;
@@ -923,10 +992,11 @@ __global__ __launch_bounds__(kFinThreads) void k_cert_bfs(CertArgs a, MultiArgs 
     uint64_t key = kEmptyKey;
     if (ck != kEmptyKey) {                       // uniform over the group
         const int32_t id = key_id(ck);
-        const float dot = qf.dot(a.emb + int64_t(id) * a.d, sub);
+        const float ts = a.ts[id];
+        const int32_t mod = (a.mod_filter >= 0) ? a.mods[id] : 0;
+        const float dot = cert_dot(qf, a.emb + int64_t(id) * a.d, sub);
         const QueryTerms t{a.t_q, a.lambda, a.mod_filter, -1, 0.0f};
-        const float sc = fuse_score(row16_sum(dot), a.ts[id], (a.mod_filter >= 0) ? a.mods[id] : 0, -1, t);
-        key = make_key(sc, uint32_t(id));
+        key = make_key(fuse_score(row16_sum(dot), ts, mod, -1, t), uint32_t(id));
     }
     if (sub == 0) s_exact[g] = key;
     __syncthreads();
@@ -1098,18 +1168,32 @@ __global__ __launch_bounds__(kFinThreads) void k_cert_bfs(CertArgs a, MultiArgs 
     }
     __syncthreads();
     stamp_at(4);
-    // exact fused scores of the marked nodes past the seeds (one per 16-lane group)
+    // exact fused scores of the marked nodes past the seeds (one per 16-lane group). A group's next
+    // four node ids are loaded together, and each row's loads go out before its first FMA (1M rows,
+    // 1,184 nodes visited: 9.1 -> 8.4 us).
     {
         QF qf;
         qf.load(a.q, sub);
         const QueryTerms t{a.t_q, a.lambda, a.mod_filter, -1, 0.0f};
-        for (int i = g; i < r; i += kFinThreads / 16) {
-            const int p = rlist[i];
-            if (p < ns) continue;                // uniform over the group
-            const int32_t id = ld_coherent(v.vlist + p);
-            const float dot = qf.dot(a.emb + int64_t(id) * a.d, sub);
-            const float sc = fuse_score(row16_sum(dot), a.ts[id], (a.mod_filter >= 0) ? a.mods[id] : 0, -1, t);
-            if (sub == 0) m.vfin[p] = sc;
+        constexpr int kGroups = kFinThreads / 16;
+        for (int i0 = g; i0 < r; i0 += 4 * kGroups) {
+            int32_t ids[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = i0 + j * kGroups;
+                const int p = i < r ? rlist[i] : 0;
+                ids[j] = p < ns ? -1 : ld_coherent(v.vlist + p);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int32_t id = ids[j];
+                if (id < 0) continue;            // uniform over the group
+                const float ts = a.ts[id];
+                const int32_t mod = (a.mod_filter >= 0) ? a.mods[id] : 0;
+                const float dot = cert_dot(qf, a.emb + int64_t(id) * a.d, sub);
+                const float sc = fuse_score(row16_sum(dot), ts, mod, -1, t);
+                if (sub == 0) m.vfin[rlist[i0 + j * kGroups]] = sc;
+            }
         }
     }
     __threadfence_block();
@@ -1199,7 +1283,7 @@ __global__ __launch_bounds__(kFinThreads) void k_cert_multi8(CertMArgs a) {
     uint64_t key = kEmptyKey;
     if (ck != kEmptyKey) {                       // uniform over the group
         const int32_t id = key_id(ck);
-        const float dot = row16_sum(qf.dot(a.emb + int64_t(id) * a.d, sub));
+        const float dot = row16_sum(cert_dot(qf, a.emb + int64_t(id) * a.d, sub));
         float sc = dot;
         if (!plain) {
             const QueryTerms t{a.tq ? a.tq[j] : a.tq_value, a.lambda, a.mod_filter, -1, 0.0f};

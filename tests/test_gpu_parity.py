@@ -483,3 +483,31 @@ def test_read_ceiling(rng):
             assert e.value.code == -5
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("k,copies", [(1, 0), (33, 70), (64, 0), (64, 1500)])
+def test_seed_merge_with_ties_and_many_keys(k, copies, rng):
+    """The finalize kernel's merge of the scan's keys: every seed count, and rows so often equal
+    (their ids order them) that the keys at or below the merge's cut outgrow one wave's sort (70)
+    and the gathering buffer (1,500)."""
+    n, d = 30_000, 256
+    emb, mods, ts, row, col, _ = random_graph(rng, n, d)
+    if copies:
+        emb[rng.choice(n, copies, replace=False)] = emb[0]
+    ts[:] = 100.0
+    dev = Dev(emb, mods, ts, row, col)
+    try:
+        mars_amd.query_memory_fast(dev.dg, dev.ctx, emb[0], T_Q, RetrievalConfig(
+            top_k=k, bfs_max_hops=1, time_decay_lambda=0.0, max_results_returned=k))
+        idx, val = dev.ctx.last_seeds()
+    finally:
+        dev.close()
+    dots = emb.astype(np.float64) @ emb[0].astype(np.float64)
+    assert len(idx) == k and len(set(idx.tolist())) == k
+    kth = np.sort(dots)[-k]
+    assert np.all(dots[idx] >= kth - 1e-5) and np.all(np.abs(val - dots[idx]) <= 1e-5)
+    pair = list(zip((-val).tolist(), idx.tolist()))
+    assert pair == sorted(pair)                          # score descending, id ascending
+    if copies:
+        same = np.flatnonzero(np.all(emb == emb[0], axis=1))
+        np.testing.assert_array_equal(idx[: min(k, len(same))], same[: min(k, len(same))])
