@@ -630,10 +630,10 @@ int32_t mm_chunk(int64_t q, int64_t n) {
 // Row ranges x query blocks for the batched scan: one 512-thread workgroup per CU
 // (256 CUs), all query blocks of a row range on one XCD.
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
-                int32_t max_ranges, int32_t kp) {
+                int32_t max_ranges, int32_t kp, bool rq64) {
     // n_qblocks counts 64-query blocks (the layout of the partial keys) for every kernel
     const int32_t qblocks = (q + 63) / 64;
-    const bool gemm = batch_uses_gemm(q, plain), rq = batch_uses_rq(q, plain);
+    const bool gemm = batch_uses_gemm(q, plain), rq = batch_uses_rq(q, plain, rq64);
     const int32_t wgq = gemm ? 256 : (rq ? 64 * batch_rq_tiles(q) : 64);   // queries per workgroup
     const int32_t tiles = (q + wgq - 1) / wgq;                             // workgroups per row range
     const int64_t align = gemm ? 256 : 16;                            // rows per tile
@@ -1552,7 +1552,9 @@ int mars_query_batch(const mars_graph* gh, mars_ctx* ch, const float* dq, int32_
     int32_t nrr = 0, nqb = 0;
     int64_t rpr = 0;
     const int32_t kp = batch_kpart(K);
-    batch_grid(n_live, Q, false, &nrr, &nqb, &rpr, 256, kp);
+    const bool uniform = std::all_of(h_tq, h_tq + Q, [&](float x) { return x == h_tq[0]; });
+    const bool rq64 = batch_small_rq(Q, n_live, uniform);
+    batch_grid(n_live, Q, false, &nrr, &nqb, &rpr, 256, kp, rq64);
     MARS_TRY(ensure_batch_scratch(c, Q, int64_t(nqb) * nrr * 64 * kp));
     hipStream_t s = c.stream;
     MARS_HIP(hipMemcpyAsync(c.btq, h_tq, size_t(Q) * sizeof(float), hipMemcpyHostToDevice, s));
@@ -1563,7 +1565,8 @@ int mars_query_batch(const mars_graph* gh, mars_ctx* ch, const float* dq, int32_
     a.emb16 = g.emb16; a.n = n_live; a.d = g.d; a.qh = c.bq; a.q = Q; a.tq = c.btq; a.ts = g.ts; a.mods = g.mods;
     a.lambda = cfg->time_decay_lambda; a.mod_filter = cfg->modality_filter; a.k = K; a.q_plain = Q; a.self_base = -1;
     a.part = c.bpart; a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
-    a.uniform_tq = std::all_of(h_tq, h_tq + Q, [&](float x) { return x == h_tq[0]; }) ? 1 : 0;
+    a.uniform_tq = uniform ? 1 : 0;
+    a.rq64 = rq64 ? 1 : 0;
     MARS_TRY(launch_batch_topk(a, K, c.bout, s, timing ? c.ev[1] : nullptr));
     if (timing) MARS_HIP(hipEventRecord(c.ev[2], s));
     std::vector<uint64_t> keys(size_t(Q) * K);
@@ -1739,7 +1742,9 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
             int32_t nrr = 0, nqb = 0;
             int64_t rpr = 0;
             const int32_t kp = batch_kpart(kMultiCand);
-            batch_grid(n_live, Qt, Qg == 0, &nrr, &nqb, &rpr, 256, kp);   // the k-NN queries alone: plain
+            const bool uniform = Qg == 0 || std::all_of(h_tq, h_tq + Qg, [&](float x) { return x == h_tq[0]; });
+            const bool rq64 = batch_small_rq(Qt, n_live, uniform);
+            batch_grid(n_live, Qt, Qg == 0, &nrr, &nqb, &rpr, 256, kp, rq64);   // the k-NN queries alone: plain
             MARS_TRY(ensure_batch_scratch(c, Qt, int64_t(nqb) * nrr * 64 * kp));
             if (Qg > 0) {
                 MARS_HIP(hipMemcpyAsync(c.btq, h_tq, size_t(Qg) * sizeof(float), hipMemcpyHostToDevice, s));
@@ -1755,7 +1760,8 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
             b.mods = g.mods; b.lambda = Qg > 0 ? lambda : 0.0f; b.mod_filter = Qg > 0 ? cfg->modality_filter : -1;
             b.k = kMultiCand; b.nrm = g.nrm; b.q_plain = Qg; b.self_base = knn_count > 0 ? knn_first : -1; b.part = c.bpart;
             b.rows_per_range = rpr; b.n_rranges = nrr; b.n_qblocks = nqb;
-            b.uniform_tq = (Qg == 0 || std::all_of(h_tq, h_tq + Qg, [&](float x) { return x == h_tq[0]; })) ? 1 : 0;
+            b.uniform_tq = uniform ? 1 : 0;
+            b.rq64 = rq64 ? 1 : 0;
             MARS_TRY(launch_batch_topk(b, kMultiCand, c.bout, s));
             if (timing) MARS_HIP(hipEventRecord(c.ev[1], s));
             if (knn_count > 0)

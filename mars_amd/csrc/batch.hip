@@ -448,7 +448,7 @@ int launch_batch_t(const BatchArgs& a, hipStream_t s) {
 template <int K>
 int launch_batch_k(const BatchArgs& a, hipStream_t s) {
     const bool plain = a.q_plain == 0;
-    if (batch_uses_rq(a.q, plain)) return launch_batch_rq(a, s);
+    if (batch_uses_rq(a.q, plain, a.rq64 != 0)) return launch_batch_rq(a, s);
     if (batch_uses_gemm(a.q, plain)) return launch_batch_mm(a, s);
     MARS_CHECK(a.floor_keys == nullptr, MARS_ERR_INVALID, "k_batch_scan takes no score floor");
     switch (a.d / 32) {
@@ -464,11 +464,16 @@ int launch_batch_k(const BatchArgs& a, hipStream_t s) {
 
 bool batch_dim_supported(int32_t d) { return d == 256 || d == 384 || d == 512 || d == 768; }
 bool batch_uses_gemm(int32_t q, bool plain) { return plain && q >= kGemmMinQ; }
-bool batch_uses_rq(int32_t q, bool plain) { return q > kRqMaxScanQ && !batch_uses_gemm(q, plain); }
-bool batch_keeps_all(int32_t q, bool plain, int64_t rows_per_range, int32_t kp) {
-    return batch_uses_rq(q, plain) && rows_per_range == kp;
+bool batch_uses_rq(int32_t q, bool plain, bool rq64) {
+    return (q > kRqMaxScanQ || rq64) && !batch_uses_gemm(q, plain);
 }
-int batch_rq_tiles(int32_t q) { return q <= 128 ? 2 : 4; }
+bool batch_small_rq(int32_t q, int64_t n, bool uniform) {
+    return q <= kRqMaxScanQ && (uniform || n <= (kRqFloorTiles - 1) * 16 * 256);
+}
+bool batch_keeps_all(const BatchArgs& a, int32_t kp) {
+    return batch_uses_rq(a.q, a.q_plain == 0, a.rq64 != 0) && a.rows_per_range == kp;
+}
+int batch_rq_tiles(int32_t q) { return q <= 64 ? 1 : q <= 128 ? 2 : 4; }
 int batch_kpart(int32_t k) { return k <= 8 ? 8 : 16; }
 
 int launch_batch_scan(const BatchArgs& a, hipStream_t s) {
@@ -516,8 +521,8 @@ int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, 
     // K (1 + ln(rows / K)) rows per range (every new best of the rows seen so far), with
     // it about rows x K / sampled rows.
     const bool gemm = batch_uses_gemm(a.q, a.q_plain == 0);
-    a.sample_pass = batch_keeps_all(a.q, a.q_plain == 0, a.rows_per_range, kp) ? 1 : 0;   // one pass, every row's key
-    const int64_t rq_rows = batch_uses_rq(a.q, a.q_plain == 0) ? rq_sample_rows(a, kp) : 0;
+    a.sample_pass = batch_keeps_all(a, kp) ? 1 : 0;   // one pass, every row's key
+    const int64_t rq_rows = batch_uses_rq(a.q, a.q_plain == 0, a.rq64 != 0) ? rq_sample_rows(a, kp) : 0;
     if (gemm || rq_rows > 0) {
         BatchArgs b = a;
         b.rows_per_range = gemm ? std::min<int64_t>(a.rows_per_range, (kMmSampleTiles + a.n_rranges - 1) / a.n_rranges * 256)

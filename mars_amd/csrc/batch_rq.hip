@@ -1,6 +1,6 @@
 // ============================================================================
 //  batch_rq.hip — k_batch_rq: batched scoring with the queries held in registers,
-//  for batches of 65 .. 1023 queries (128 or 256 per workgroup, one corpus pass each).
+//  for batches of up to 1023 queries (64, 128 or 256 per workgroup, one corpus pass each).
 //
 //  A query tile of 256 fp16 queries x d does not fit in LDS (384 KiB at d = 768), but
 //  it fits in the register files of one CU: each of the four waves (one per SIMD, the
@@ -85,12 +85,12 @@ __device__ __attribute__((always_inline)) inline void dma4(const void* g, uint32
 
 // Workgroups per query group of a launch that keeps every row: one tile each, at most 256 in all.
 __host__ __device__ inline int rq_all_wgs(const BatchArgs& a) {
-    const int wgq = a.q <= 128 ? 128 : 256, groups = (a.q + wgq - 1) / wgq;
+    const int wgq = a.q <= 64 ? 64 : a.q <= 128 ? 128 : 256, groups = (a.q + wgq - 1) / wgq;
     const int64_t tiles = (a.n + kRRows - 1) / kRRows, most = 256 / groups > 1 ? 256 / groups : 1;
     return int(tiles < most ? tiles : most);
 }
 
-// QT: 16-query MFMA tiles per wave (2 or 4: 128 or 256 queries per workgroup). MODE: the
+// QT: 16-query MFMA tiles per wave (1, 2 or 4: 64, 128 or 256 queries per workgroup). MODE: the
 // full pass keeps the best K keys per query and range; the sampled pass of launch_batch_topk
 // keeps K row-class maxima instead; kRqAll writes every row's key (batch_keeps_all).
 constexpr int kRqFull = 0, kRqSample = 1, kRqAll = 2;
@@ -555,7 +555,11 @@ int launch_rq_q(const BatchArgs& a, hipStream_t s) {
 
 template <int NS, int K>
 int launch_rq_t(const BatchArgs& a, hipStream_t s) {
-    return batch_rq_tiles(a.q) == 2 ? launch_rq_q<NS, K, 2>(a, s) : launch_rq_q<NS, K, 4>(a, s);
+    switch (batch_rq_tiles(a.q)) {
+        case 1: return launch_rq_q<NS, K, 1>(a, s);
+        case 2: return launch_rq_q<NS, K, 2>(a, s);
+        default: return launch_rq_q<NS, K, 4>(a, s);
+    }
 }
 
 template <int K>

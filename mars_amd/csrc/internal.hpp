@@ -89,7 +89,7 @@ void dfree(T*& p) {
 // per query and range the launch keeps (batch_kpart), or 0; with it a k_batch_rq launch of few
 // rows gets ranges of kp rows, which keep every row (batch_keeps_all).
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
-                int32_t max_ranges = 256, int32_t kp = 0);
+                int32_t max_ranges = 256, int32_t kp = 0, bool rq64 = false);
 
 constexpr int kMaxK = 64;              // seeds per query (wave-held list), as MAX_TOP_K
 constexpr int kSortCap = 8192;         // results sorted in LDS by the finalize kernel (one band)
@@ -535,6 +535,7 @@ struct BatchArgs {
     int32_t n_rranges;
     int32_t n_qblocks;
     int32_t uniform_tq;      // all query times equal: one decay weight per row
+    int32_t rq64;            // up to 64 queries: k_batch_rq, not k_batch_scan (batch_small_rq)
     int32_t sample_pass;     // the sampled pass of launch_batch_topk: its keys serve only as
                              // floors (k_batch_mm then keeps group maxima, not the best K)
 };
@@ -578,7 +579,15 @@ int32_t mm_ranges(int32_t groups, int64_t tiles);
 int32_t mm_chunk(int64_t q, int64_t n);
 constexpr int32_t kRqMaxScanQ = 64;
 bool batch_uses_gemm(int32_t q, bool plain);
-bool batch_uses_rq(int32_t q, bool plain);
+// rq64: a batch of up to 64 queries may take k_batch_rq too (BatchArgs::rq64)
+bool batch_uses_rq(int32_t q, bool plain, bool rq64);
+// Whether a batch of up to 64 queries takes k_batch_rq (one 16-query tile per wave) rather than
+// k_batch_scan: with one query time, or where every row's key is kept. (The whole call, k_batch_scan
+// / k_batch_rq: 64 queries over 1M rows of 768, one time 347 / 323 us, per-query times and decay
+// 374 / 392; 17 over 300K 139 / 137 and 142 / 166; 64 over 30,000 88 / 65 and 90 / 67; 1 over 6,000
+// 65 / 43 us. Inserts' neighbour searches stay with k_batch_scan, which leaves a CU's LDS to
+// the queries beside them.)
+bool batch_small_rq(int32_t q, int64_t n, bool uniform);
 // A k_batch_rq launch whose ranges hold as many rows as keys: its product is written whole, a
 // key per row, and the merge selects. batch_grid lays launches out so where a workgroup would have
 // fewer than kRqFloorTiles tiles: there a floor's passes (rq_sample_rows) and filling and searching
@@ -586,7 +595,7 @@ bool batch_uses_rq(int32_t q, bool plain);
 // over 6,307 rows, 4 tiles, 90 / 74 us; 512 over 12,000, 6 tiles, 117 / 90; 256 over 40,000, 10
 // tiles, 122 / 110; 100 over 50,000, 13 tiles, 98 / 98; 80 over 60,000, 15 tiles, 88 / 106 us.)
 constexpr int64_t kRqFloorTiles = 12;
-bool batch_keeps_all(int32_t q, bool plain, int64_t rows_per_range, int32_t kp);
+bool batch_keeps_all(const BatchArgs& a, int32_t kp);
 int batch_rq_tiles(int32_t q);   // 16-query MFMA tiles per k_batch_rq wave: 2 or 4
 int launch_batch_rq(const BatchArgs& a, hipStream_t s);
 int batch_kpart(int32_t k);  // keys per (query, row range) the scan writes

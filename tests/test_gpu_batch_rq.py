@@ -216,3 +216,27 @@ def test_merge_of_few_and_many_keys(n, q, k, rng):
     np.testing.assert_array_equal(ids, np.tile(want, (q, 1)))
     live = want >= 0
     assert np.all(sc[:, live] == sc[0, 0]) and abs(sc[0, 0] - 1.0) < 2e-3
+
+
+@pytest.mark.parametrize("d", [256, 768])
+@pytest.mark.parametrize("q,k,filt", [(1, 8, -1), (15, 16, 1), (17, 3, -1), (63, 10, 2)])
+def test_small_uniform_batch_equals_scan_bit_for_bit(d, q, k, filt, rng):
+    """Up to 64 queries of one time take k_batch_rq; with one more query of another time the batch
+    takes k_batch_scan (50,000 rows: more than are kept whole). Same ids and score bits."""
+    n = 50_000
+    emb, mods, ts, _, _, _ = random_graph(rng, n, d)
+    emb[100:130] = emb[100]
+    dev = Dev(emb, mods, ts, None, None, fp16=True)
+    qs = np.ascontiguousarray(emb[np.r_[100, rng.choice(n, q, replace=False)]])
+    tq = np.full(q + 1, T_Q, np.float32)
+    tq[q] -= 50.0
+    cfg = RetrievalConfig(top_k=k, time_decay_lambda=LAM, modality_filter=filt)
+    buf = mars_amd.DeviceBuffer.from_array(qs)
+    try:
+        ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq[:q], cfg)
+        ids2, sc2 = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q + 1, tq, cfg)
+    finally:
+        buf.free()
+        dev.close()
+    np.testing.assert_array_equal(ids, ids2[:q])
+    np.testing.assert_array_equal(sc.view(np.uint32), sc2[:q].view(np.uint32))
