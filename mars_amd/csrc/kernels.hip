@@ -1283,7 +1283,7 @@ __global__ __launch_bounds__(kFinThreads) void k_cert_multi8(CertMArgs a) {
     uint64_t key = kEmptyKey;
     if (ck != kEmptyKey) {                       // uniform over the group
         const int32_t id = key_id(ck);
-        const float dot = row16_sum(cert_dot(qf, a.emb + int64_t(id) * a.d, sub));
+        const float dot = row16_sum(qf.dot(a.emb + int64_t(id) * a.d, sub));
         float sc = dot;
         if (!plain) {
             const QueryTerms t{a.tq ? a.tq[j] : a.tq_value, a.lambda, a.mod_filter, -1, 0.0f};
