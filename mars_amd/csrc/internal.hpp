@@ -541,21 +541,19 @@ struct BatchArgs {
 };
 bool batch_dim_supported(int32_t d);
 // Three kernels score a batch, by its size and kind (1M rows, d = 768, one MI355X):
-//   Q <= kRqMaxScanQ              k_batch_scan: 64-query blocks, rows streamed into
-//                                 registers (Q = 64: 313 us);
+//   Q <= kRqMaxScanQ              k_batch_scan: 64-query blocks, rows streamed into registers
+//                                 (Q = 64: 310 us); or, with one query time or few rows,
+//                                 k_batch_rq (batch_small_rq)
 //   Q > kRqMaxScanQ               k_batch_rq (batch_rq.hip): the queries held in registers
-//                                 (128 or 256 per workgroup, batch_rq_tiles x 16 per wave),
+//                                 (64, 128 or 256 per workgroup, batch_rq_tiles x 16 per wave),
 //                                 16-row tiles streamed through LDS, a sampled score floor
-//                                 (Q = 256: 485 us the whole call);
+//                                 (Q = 256: full pass 375-390 us)
 //   neighbour searches, Q >= kGemmMinQ
 //                                 k_batch_mm: 256-query x 256-row LDS tiles, thresholds from
-//                                 the sampled floor (the k-NN builders' 1024-query chunks:
-//                                 1.90 ms, against 2.86 ms through k_batch_rq). With decayed
-//                                 scores its raw-dot thresholds pass far more rows than reach
-//                                 the lists, and k_batch_rq is faster (Q = 1024: 1.80 against
-//                                 2.50 ms).
-// (With 64 queries per workgroup k_batch_rq measured slower than the scan: 445 against
-// 408 us on a random 1M corpus.)
+//                                 the sampled floor (chunks of 1024 queries 1.90 ms, against 2.86
+//                                 ms through k_batch_rq, both as first built). With decayed scores
+//                                 its raw-dot thresholds pass far more rows than reach the lists,
+//                                 and k_batch_rq is faster (Q = 1024: 1.80 against 2.50 ms then).
 constexpr int32_t kGemmMinQ = 1024;
 // k_batch_mm's grid: groups of 256 queries x row ranges of 256-row tiles, one workgroup each
 // and one per CU. mm_xcd_groups: the XCDs a launch's groups are split over, the fewest that

@@ -1,16 +1,17 @@
-"""GPU parity of the batched scoring kernel for 65 .. 1023 queries (k_batch_rq: 128 or 256
-queries per workgroup in registers, 16-row tiles through LDS, a sampled score floor).
+"""GPU parity of k_batch_rq (batched scoring with 64, 128 or 256 queries per workgroup in
+registers, 16-row tiles through LDS, a sampled score floor).
 
 - against the fp32 oracle's top-K (the bar of tests/parity.py: scores within 2e-3 of the
   scale, id sets equal up to near-ties) at every supported width, both list sizes, with
   and without a modality filter, one or per-query times, ragged row counts;
-- bit for bit against k_batch_scan (batches of at most 64 queries), which computes the
-  same MFMA products in the same order: the same queries scored in one batch (256, 128 or
-  96 queries) and in batches of 32 give the same ids and scores;
-- with a corpus large enough that each row range is sampled for the score floor, against
-  the oracle and bit for bit against batches of 32 (which take no floor);
+- bit for bit against k_batch_scan, which computes the same MFMA products in the same order: on
+  more rows than are kept whole (45,056), batches of up to 64 queries with per-query times take
+  it, and with one time k_batch_rq; batches of 32 of fewer rows or one time are k_batch_rq's
+  form for up to 64 queries, against its 128- and 256-query forms;
+- floors, lists, tiles with many and few passing rows, and the form that keeps every row;
 - the neighbour-search form (plain dot products, the node itself excluded) against the
-  exact CPU k-NN.
+  exact CPU k-NN;
+- the merge of the ranges' keys.
 """
 from __future__ import annotations
 
@@ -55,7 +56,7 @@ def test_rq_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
     try:
         ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # k_batch_rq
         parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, 32, tq[j:j + 32], cfg)
-                 for j in range(0, q, 32)]                                                   # k_batch_scan
+                 for j in range(0, q, 32)]
     finally:
         buf.free()
         dev.close()
@@ -85,7 +86,7 @@ def test_rq_sampled_floor(rng):
 def test_rq_sampled_floor_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
     """The sampled floor drops no row that belongs in a list: on 200K rows (each 256-query
     group's ranges sampled for the floor), the batch's ids and score bits equal those of
-    the same queries scored in batches of 32 by k_batch_scan (no floor), with a modality
+    the same queries scored in batches of 32 (k_batch_scan, which takes no floor, with per-query times), with a modality
     filter and with per-query times too."""
     n, d = 200_000, 256
     emb = rng.standard_normal((n, d)).astype(np.float32)
@@ -100,7 +101,7 @@ def test_rq_sampled_floor_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
     try:
         ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # sampled floor
         parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, min(32, q - j), tq[j:j + 32], cfg)
-                 for j in range(0, q, 32)]                                                   # k_batch_scan
+                 for j in range(0, q, 32)]
     finally:
         buf.free()
         dev.close()
@@ -185,7 +186,7 @@ def test_rq_floors_and_queues_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng)
     try:
         ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # k_batch_rq
         parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, min(32, q - j), tq[j:j + 32], cfg)
-                 for j in range(0, q, 32)]                                                   # k_batch_scan
+                 for j in range(0, q, 32)]
     finally:
         buf.free()
         dev.close()
