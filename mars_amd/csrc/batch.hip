@@ -517,9 +517,8 @@ int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, 
     a.range_stride = 0;
     a.floor_keys = nullptr;
     a.floor_k = 0;
-    // The floor pays where a range is long: without it a query inserts about
-    // K (1 + ln(rows / K)) rows per range (every new best of the rows seen so far), with
-    // it about rows x K / sampled rows.
+    // Without a floor a query inserts about K (1 + ln(rows / K)) rows per range (every new best of
+    // the rows seen so far), with it about rows x K / sampled rows.
     const bool gemm = batch_uses_gemm(a.q, a.q_plain == 0);
     a.sample_pass = batch_keeps_all(a, kp) ? 1 : 0;   // one pass, every row's key
     const int64_t rq_rows = batch_uses_rq(a.q, a.q_plain == 0, a.rq64 != 0) ? rq_sample_rows(a, kp) : 0;

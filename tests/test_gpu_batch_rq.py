@@ -66,7 +66,7 @@ def test_rq_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
 
 def test_rq_sampled_floor(rng):
     """200K rows, 600 queries (three 256-query groups over 80 row ranges of 2,512 rows):
-    each range's first sixty-fourth (32 rows) is scored first and sets the queries' floors."""
+    each range's first tiles are scored first and set the queries' floors."""
     n, d = 200_000, 256
     emb = rng.standard_normal((n, d)).astype(np.float32)
     emb /= np.linalg.norm(emb, axis=1, keepdims=True)
