@@ -518,7 +518,8 @@ void k_batch_rq(BatchArgs a) {
     __builtin_amdgcn_s_waitcnt(rq_wait_vm(0));
     if constexpr (MODE == kRqSample) {
         // K distinct rows' scores per query and range: the maxima of the 16 row classes, or (K = 8)
-        // of the class pairs m, m + 8; keyed with the class (only the score is used)
+        // of the class pairs m, m + 8; keyed with the class (only the score is used). A class without
+        // a score above -inf (no rows, or NaN alone, which ranks below -inf) is no row to count.
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
@@ -528,7 +529,7 @@ void k_batch_rq(BatchArgs a) {
                 if constexpr (K == 8) x = fmaxf(x, xor_lanef<8>(x));
                 if (qi < a.q && m < K)
                     a.part[((int64_t(qi / 64) * a.n_rranges + r_id) * 64 + qi % 64) * K + m] =
-                        make_key(x, uint32_t(r0) + uint32_t(m));
+                        x > -INFINITY ? make_key(x, uint32_t(r0) + uint32_t(m)) : kEmptyKey;
             }
     } else if constexpr (FULL) {
         if (qvalid) {

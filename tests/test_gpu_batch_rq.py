@@ -241,3 +241,38 @@ def test_small_uniform_batch_equals_scan_bit_for_bit(d, q, k, filt, rng):
         dev.close()
     np.testing.assert_array_equal(ids, ids2[:q])
     np.testing.assert_array_equal(sc.view(np.uint32), sc2[:q].view(np.uint32))
+
+
+@pytest.mark.parametrize("q,k,uniform", [(40, 8, True), (70, 10, False), (130, 16, False), (300, 5, True), (600, 16, False)])
+def test_nan_query_with_sampled_floors(q, k, uniform, rng):
+    """A query whose every score is NaN (which ranks below -inf) in a batch with floors (50,000 rows:
+    at least 12 tiles per workgroup): its sampled rows set no floor, and it gets the least ids, as from
+    a scan without floors; the other queries' answers stay. So does a node of a NaN row in a range of
+    neighbour searches."""
+    n, d = 50_000, 256
+    emb, mods, ts, _, _, _ = random_graph(rng, n, d)
+    bad = 20_000 + q // 2
+    emb[bad, 9] = np.nan
+    dev = Dev(emb, mods, ts, None, None, fp16=True)
+    qs = np.ascontiguousarray(emb[rng.choice(20_000, q, replace=False)])
+    tq = np.full(q, T_Q, np.float32) if uniform else rng.uniform(300, 600, q).astype(np.float32)
+    cfg = RetrievalConfig(top_k=k, time_decay_lambda=LAM)
+    try:
+        out = []
+        for at in (None, 2, q - 1):
+            x = qs.copy()
+            if at is not None:
+                x[at, 3] = np.nan
+            buf = mars_amd.DeviceBuffer.from_array(x)
+            out.append(mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg))
+            buf.free()
+        knn = mars_amd.graph_knn_range(dev.dg, 8, 20_000, q)
+    finally:
+        dev.close()
+    for at, (ids, sc) in zip((2, q - 1), out[1:]):
+        np.testing.assert_array_equal(ids[at], np.arange(k))
+        assert np.all(np.isnan(sc[at]))
+        rest = np.arange(q) != at
+        np.testing.assert_array_equal(ids[rest], out[0][0][rest])
+        np.testing.assert_array_equal(sc[rest].view(np.uint32), out[0][1][rest].view(np.uint32))
+    np.testing.assert_array_equal(knn[bad - 20_000], np.arange(8))
