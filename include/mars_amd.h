@@ -443,7 +443,7 @@ int mars_query_batch(const mars_graph* g, mars_ctx* ctx, const float* d_queries,
 /* mars_query_batch without allocation. No counterpart in the reference: for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops). The
  * same kernels and results as mars_query_batch, with their scratch in a static device
- * array of the library (about 8.4 MiB, held per GPU until the process ends): Q <= 256
+ * array of the library (about 48.4 MiB, held per GPU until the process ends): Q <= 256
  * queries (MARS_ERR_CAPACITY beyond), top_k <= 16, embedding_dim 256 / 384 / 512 / 768.
  * Inputs and outputs are device memory: d_queries Q x embedding_dim fp32, d_tq Q query
  * times (uniform_tq != 0 promises they are all equal: one decay weight per row), d_ids /

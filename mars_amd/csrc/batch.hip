@@ -503,7 +503,7 @@ namespace {
 constexpr double kRqHitTiles = 1.0 / 20;
 int64_t rq_sample_rows(const BatchArgs& a, int32_t kp) {
     const int64_t tiles = a.rows_per_range / 16;
-    if (tiles < kRqFloorTiles) return 0;
+    if (tiles < kRqListTiles) return 0;
     const double s = std::sqrt(kRqHitTiles * 16 * batch_rq_tiles(a.q) * kp * double(tiles) / a.n_rranges);
     return 16 * std::min<int64_t>(std::max<int64_t>(1, int64_t(s + 0.5)), tiles / 2);
 }

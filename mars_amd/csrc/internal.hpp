@@ -593,6 +593,13 @@ bool batch_small_rq(int32_t q, int64_t n, bool uniform);
 // over 6,307 rows, 4 tiles, 90 / 74 us; 512 over 12,000, 6 tiles, 117 / 90; 256 over 40,000, 10
 // tiles, 122 / 110; 100 over 50,000, 13 tiles, 98 / 98; 80 over 60,000, 15 tiles, 88 / 106 us.)
 constexpr int64_t kRqFloorTiles = 12;
+// 48 MiB of keys (one per query and row; the lists' layout needs 32 KiB per query at most, whatever the rows).
+constexpr int64_t kRqAllKeys = int64_t(6) << 20;
+// Ranges of fewer tiles than this keep lists without a floor, whose pass over 1 tile of 2 or 3 costs
+// what it saves. (Lists of short ranges are k_batch_rq's slowest form: the whole call without / with a
+// floor, one query time: 256 queries over 40,000 rows, 10 tiles, 183 / 94 us; over 24,000, 6 tiles, 128 / 86;
+// 4 tiles 98 / 81; 3 tiles 83 / 77 and, over 8,000, 2 tiles, 69 / 77.)
+constexpr int64_t kRqListTiles = 4;
 bool batch_keeps_all(const BatchArgs& a, int32_t kp);
 int batch_rq_tiles(int32_t q);   // 16-query MFMA tiles per k_batch_rq wave: 2 or 4
 int launch_batch_rq(const BatchArgs& a, hipStream_t s);

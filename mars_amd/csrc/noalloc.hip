@@ -3,8 +3,9 @@
 //  nothing, for callers that cannot call hipMalloc (code under HIP graph capture,
 //  tight serving loops).
 //
-//  The same kernels as mars_query_batch (fp32 -> fp16 query rows, k_batch_scan,
-//  k_batch_merge), with their scratch in one file-scope device array instead of
+//  The same kernels as mars_query_batch (fp32 -> fp16 query rows, k_batch_rq, k_batch_merge; up
+//  to 64 queries always k_batch_scan, which neither takes a CU's whole LDS and registers from the
+//  work that a captured call runs beside nor adds a floor's two launches), with their scratch in one file-scope device array instead of
 //  context buffers: the queries' fp16 rows, the per-row-range partial keys and
 //  the merged keys. The device address of that array is taken once per device
 //  with hipGetSymbolAddress, at set-up (mars_init, and mars_graph_create on the
@@ -28,11 +29,13 @@ namespace {
 constexpr int32_t kStaticMaxQ = 256;                      // queries per call
 constexpr int32_t kStaticMaxD = 768;                      // widest batched row (batch_dim_supported)
 constexpr size_t kStaticQBytes = size_t(kStaticMaxQ) * kStaticMaxD * sizeof(__half);     // 384 KiB
-constexpr size_t kStaticPartKeys = size_t(1) << 20;      // 8 MiB of partial keys
+// 48 MiB of partial keys: every row's, wherever mars_query_batch keeps them. (With 8 MiB, which the
+// lists of any 256 queries fit, 256 queries over 12,000 rows took 83 us as lists, 55 us so.)
+constexpr size_t kStaticPartKeys = size_t(kRqAllKeys);
 constexpr size_t kStaticOutKeys = size_t(kStaticMaxQ) * 16;
 constexpr size_t kStaticPartOff = (kStaticQBytes + 255) / 256 * 256;
 constexpr size_t kStaticOutOff = kStaticPartOff + kStaticPartKeys * sizeof(uint64_t);
-constexpr size_t kStaticBytes = kStaticOutOff + kStaticOutKeys * sizeof(uint64_t);    // ~8.4 MiB
+constexpr size_t kStaticBytes = kStaticOutOff + kStaticOutKeys * sizeof(uint64_t);    // ~48.4 MiB
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];

@@ -26,6 +26,22 @@ from parity import LAM, T_Q, Dev, batch_check, random_graph
 pytestmark = pytest.mark.gpu
 
 
+def static_batch(dg, qs, tq, cfg, uniform, block=None):
+    """mars_query_batch_static in blocks of `block` queries; up to 64 of them take k_batch_scan."""
+    out = []
+    for j in range(0, len(qs), block or len(qs)):
+        x, t = np.ascontiguousarray(qs[j:j + (block or len(qs))]), np.ascontiguousarray(tq[j:j + (block or len(qs))])
+        bufs = [mars_amd.DeviceBuffer.from_array(x), mars_amd.DeviceBuffer.from_array(t),
+                mars_amd.DeviceBuffer(len(x) * cfg.top_k * 4), mars_amd.DeviceBuffer(len(x) * cfg.top_k * 4)]
+        mars_amd.query_batch_static(dg, bufs[0].ptr, len(x), bufs[1].ptr, cfg, bufs[2].ptr, bufs[3].ptr, uniform_tq=uniform)
+        mars_amd.synchronize()
+        out.append((bufs[2].to_array(np.int32, len(x) * cfg.top_k).reshape(len(x), -1),
+                    bufs[3].to_array(np.float32, len(x) * cfg.top_k).reshape(len(x), -1)))
+        for b in bufs:
+            b.free()
+    return np.concatenate([o[0] for o in out]), np.concatenate([o[1] for o in out])
+
+
 @pytest.mark.parametrize("d,q,k,filt,uniform", [(256, 129, 5, -1, True), (384, 200, 16, 1, False),
                                                  (512, 256, 8, 2, True), (768, 300, 10, -1, False),
                                                  (768, 520, 16, 0, True), (256, 1000, 3, -1, True),
@@ -276,3 +292,24 @@ def test_nan_query_with_sampled_floors(q, k, uniform, rng):
         np.testing.assert_array_equal(ids[rest], out[0][0][rest])
         np.testing.assert_array_equal(sc[rest].view(np.uint32), out[0][1][rest].view(np.uint32))
     np.testing.assert_array_equal(knn[bad - 20_000], np.arange(8))
+
+
+# ranges of 7 and 11 tiles, of more keys than are kept whole
+@pytest.mark.parametrize("q,n,k,uniform", [(256, 24_700, 5, True), (256, 45_000, 16, False), (230, 28_001, 10, False)])
+def test_static_short_ranges_equal_scan_bit_for_bit(q, n, k, uniform, rng):
+    """Batches of the static entry point whose short ranges keep lists with a floor, against
+    k_batch_scan: same ids and score bits."""
+    d = 256
+    emb, mods, ts, _, _, _ = random_graph(rng, n, d)
+    emb[100:140] = emb[100]
+    dev = Dev(emb, mods, ts, None, None, fp16=True)
+    qs = emb[np.r_[100, rng.choice(n, q - 1, replace=False)]]
+    tq = np.full(q, T_Q, np.float32) if uniform else rng.uniform(300, 600, q).astype(np.float32)
+    cfg = RetrievalConfig(top_k=k, time_decay_lambda=LAM, modality_filter=-1 if uniform else 1)
+    try:
+        ids, sc = static_batch(dev.dg, qs, tq, cfg, uniform)
+        ids2, sc2 = static_batch(dev.dg, qs, tq, cfg, uniform, 32)
+    finally:
+        dev.close()
+    np.testing.assert_array_equal(ids, ids2)
+    np.testing.assert_array_equal(sc.view(np.uint32), sc2.view(np.uint32))
