@@ -436,7 +436,9 @@ int mars_query_device(const mars_graph* g, mars_ctx* ctx, const float* d_query, 
  * fp16 tiles with fp32 accumulation. No BFS, no episode scope: each row of the
  * output is the seed list the Q=1 global path would select (scores within the fp16
  * tolerance). out_ids / out_scores: host, Q x top_k, each row sorted (score desc,
- * id asc). Reference analogue: none (wmma_similarity.cu:55-138 scores one query). */
+ * id asc). The context keeps the scratch: 16-bit rows, a time and 16 keys per query, and at
+ * most 48 MiB or 32 KiB per query of partial keys, whichever is more.
+ * Reference analogue: none (wmma_similarity.cu:55-138 scores one query). */
 int mars_query_batch(const mars_graph* g, mars_ctx* ctx, const float* d_queries, int32_t Q,
                      const float* t_q, const mars_retrieval_config* cfg, int32_t* out_ids,
                      float* out_scores, mars_stats* stats);

@@ -627,6 +627,10 @@ int32_t mm_chunk(int64_t q, int64_t n) {
     return int32_t(steps(8192) < steps(even) ? 8192 : even);
 }
 
+int64_t batch_part_room(int64_t held, int64_t need) {
+    return std::max(need, std::min(2 * held, kRqAllKeys));
+}
+
 // Row ranges x query blocks for the batched scan: one 512-thread workgroup per CU
 // (256 CUs), all query blocks of a row range on one XCD.
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
@@ -644,7 +648,9 @@ void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n
     if (rr > max_rr) rr = int32_t(max_rr);
     *n_qblocks = qblocks;
     *rows_per_range = ((n + rr - 1) / rr + align - 1) / align * align;
-    if (rq && kp > 0 && *rows_per_range < kRqFloorTiles * align) *rows_per_range = kp;
+    if (rq && kp > 0 && *rows_per_range < kRqFloorTiles * align &&
+        int64_t(qblocks) * 64 * ((n + kp - 1) / kp * kp) <= kRqAllKeys)
+        *rows_per_range = kp;
     *n_rranges = int32_t((n + *rows_per_range - 1) / *rows_per_range);
 }
 
@@ -694,10 +700,12 @@ int ensure_batch_scratch(Ctx& c, int32_t q, int64_t part_keys) {
         c.bcap_q = q;
     }
     if (part_keys > c.bcap_part) {
+        const int64_t held = c.bcap_part;
         dfree(c.bpart);
         c.bcap_part = 0;
-        MARS_TRY(dmalloc(&c.bpart, size_t(part_keys)));
-        c.bcap_part = part_keys;
+        const int64_t room = batch_part_room(held, part_keys);
+        MARS_TRY(dmalloc(&c.bpart, size_t(room)));
+        c.bcap_part = room;
     }
     return MARS_OK;
 }

@@ -87,9 +87,14 @@ void dfree(T*& p) {
 // is a neighbour search (BatchArgs::q_plain == 0), which picks the kernel as in
 // batch_uses_gemm. max_ranges caps the row ranges (workgroups per 64-query block). kp: the keys
 // per query and range the launch keeps (batch_kpart), or 0; with it a k_batch_rq launch of few
-// rows gets ranges of kp rows, which keep every row (batch_keeps_all).
+// rows gets ranges of kp rows, which keep every row (batch_keeps_all), while their keys number at most
+// kRqAllKeys.
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
                 int32_t max_ranges = 256, int32_t kp = 0, bool rq64 = false);
+// The keys a scratch that held `held` of them and must hold `need` is given: twice as many as before,
+// up to kRqAllKeys. (With every row's key kept, need follows the row count of a growing graph: exact
+// sizes would be allocated again, and the device waited for, every few inserts.)
+int64_t batch_part_room(int64_t held, int64_t need);
 
 constexpr int kMaxK = 64;              // seeds per query (wave-held list), as MAX_TOP_K
 constexpr int kSortCap = 8192;         // results sorted in LDS by the finalize kernel (one band)
@@ -593,7 +598,8 @@ bool batch_small_rq(int32_t q, int64_t n, bool uniform);
 // over 6,307 rows, 4 tiles, 90 / 74 us; 512 over 12,000, 6 tiles, 117 / 90; 256 over 40,000, 10
 // tiles, 122 / 110; 100 over 50,000, 13 tiles, 98 / 98; 80 over 60,000, 15 tiles, 88 / 106 us.)
 constexpr int64_t kRqFloorTiles = 12;
-// 48 MiB of keys (one per query and row; the lists' layout needs 32 KiB per query at most, whatever the rows).
+// At most 48 MiB of keys (one per query and row; the lists' layout needs 32 KiB per query at most,
+// whatever the rows).
 constexpr int64_t kRqAllKeys = int64_t(6) << 20;
 // Ranges of fewer tiles than this keep lists without a floor, whose pass over 1 tile of 2 or 3 costs
 // what it saves. (Lists of short ranges are k_batch_rq's slowest form: the whole call without / with a

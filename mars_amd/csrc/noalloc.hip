@@ -106,7 +106,6 @@ extern "C" int mars_query_batch_static(const mars_graph* gh, const float* d_quer
     int64_t rpr = 0;
     const int32_t kp = batch_kpart(K);
     batch_grid(n_live, Q, false, &nrr, &nqb, &rpr, 256, kp);
-    if (int64_t(nqb) * nrr * 64 * kp > int64_t(kStaticPartKeys)) batch_grid(n_live, Q, false, &nrr, &nqb, &rpr);
     const int64_t part_keys = int64_t(nqb) * nrr * 64 * kp;
     MARS_CHECK(part_keys <= int64_t(kStaticPartKeys), MARS_ERR_CAPACITY,
                "mars_query_batch_static: %lld partial keys exceed the static %zu", (long long)part_keys,
