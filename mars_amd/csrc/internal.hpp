@@ -85,8 +85,8 @@ void dfree(T*& p) {
 
 // Row ranges x query blocks of the batched scan (defined in api.hip). plain: every query
 // is a neighbour search (BatchArgs::q_plain == 0), which picks the kernel as in
-// batch_uses_gemm. max_ranges caps the row ranges (workgroups per 64-query block). kp: the keys
-// per query and range the launch keeps (batch_kpart), or 0; with it a k_batch_rq launch of few
+// batch_uses_gemm. max_ranges caps the row ranges (workgroups per 64-query block). kp (without a
+// cap): the keys per query and range the launch keeps (batch_kpart), or 0; with it a k_batch_rq launch of few
 // rows gets ranges of kp rows, which keep every row (batch_keeps_all), while their keys number at most
 // kRqAllKeys.
 void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
@@ -95,6 +95,8 @@ void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n
 // up to kRqAllKeys. (With every row's key kept, need follows the row count of a growing graph: exact
 // sizes would be allocated again, and the device waited for, every few inserts.)
 int64_t batch_part_room(int64_t held, int64_t need);
+// The same for an insert's neighbour search of q new nodes (insert.hip): few ranges, lists only.
+void insert_grid(int64_t n, int32_t q, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range);
 
 constexpr int kMaxK = 64;              // seeds per query (wave-held list), as MAX_TOP_K
 constexpr int kSortCap = 8192;         // results sorted in LDS by the finalize kernel (one band)

@@ -1,5 +1,6 @@
 """Layouts of the batched scoring's partial keys (mars::batch_grid), on the CPU: their number is bounded over
-every batch size and row count, and a growing graph's scratch is allocated a bounded number of times."""
+every batch size and row count, a growing graph's scratch is allocated a bounded number of times, and an
+insert's search keeps to its share of the chip."""
 from __future__ import annotations
 
 import ctypes as C
@@ -60,3 +61,15 @@ def test_growing_graph_allocates_a_few_times(so):
             held, times = so._ZN4mars15batch_part_roomEll(C.c_int64(held), C.c_int64(need)), times + 1
             assert need <= held <= max(ALL_KEYS, need)
     assert times <= 12
+
+
+@pytest.mark.parametrize("q", [1, 64, 65, 128, 200, 900, 1023, 1024])
+def test_inserts_keep_to_a_quarter_of_the_chip(so, q):
+    """At most 64 ranges per query group, whose buffer does not grow with the graph."""
+    f = so._ZN4mars11insert_gridEliPiS0_Pl
+    f.restype = None
+    for n in ROWS:
+        rr, qb, rows = C.c_int32(), C.c_int32(), C.c_int64()
+        f(C.c_int64(n), C.c_int32(q), C.byref(rr), C.byref(qb), C.byref(rows))
+        assert rr.value * rows.value >= n and (rr.value - 1) * rows.value < n
+        assert rr.value <= (64 if n <= 2_000_000 else 256), (n, q, rr.value)
