@@ -293,6 +293,8 @@ void k_batch_rq(BatchArgs a) {
     // the row passes unless x weight + offset < the query's bound (NaN passes). A wave of both
     // global queries and neighbour searches (whose score is x) takes every tile to select_tile.
     f32x4 tacc[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) tacc[qt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float tw = 0.0f, tb = 0.0f, tsc = 0.0f;
     bool tkeep = false;
     const bool all_plain = wq0 >= a.q_plain, mixed = !all_plain && wq0 + WQ > a.q_plain;
@@ -420,7 +422,7 @@ void k_batch_rq(BatchArgs a) {
     for (int i = 0; i < ntiles + (FULL ? 1 : 0); ++i) {
         const int t0 = r0 + i * kRRows;
         uint64_t hits = ~0ull;                   // lanes whose row reached a bound in the tile under test
-        f32x4 acc[QT];
+        f32x4 acc[QT] = {};
         float sts = 0.0f;
         bool keep_m = false;
         if (i < ntiles) {
