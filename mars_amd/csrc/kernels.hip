@@ -595,10 +595,12 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(FinalizeArgs a) {
     // Every key of the K best is <= the scan's final bound (the smallest workgroup K-th
     // key), so keys above it are dropped as they load and never reach the lists.
     const uint64_t gb = *a.gthr;
-    // The keys in 64 columns (the lanes of all waves): k keys are <= the k-th least of the columns'
-    // least keys, so only keys at or below that cut are gathered and sorted, about k ln(64 / (64 -
-    // k)) 64 / k of them (45 at k = 32). (Sorting every 64 keys into each wave's list bounded this by
-    // issue: k = 32 of 512 workgroups' keys 24 -> 5 us.)
+    // Up to one key per thread: each wave sorts its 64, and the waves' lists are merged. More: the keys
+    // in 64 columns (the lanes of all waves): k keys are <= the k-th least of the columns' least keys,
+    // so only keys at or below that cut are gathered and sorted, about k ln(64 / (64 - k)) 64 / k of
+    // them (45 at k = 32). (Sorting every 64 keys into each wave's list bounded this by issue: k = 32
+    // of 512 workgroups' keys 24 -> 5 us. The cut's barriers and its own sort take longer than one
+    // sort per wave: the whole call at k = 1 over 2,000 rows 27.7 -> 24.8 us, over 10,000 29.8 -> 27.2.)
     uint64_t x[8], least = kEmptyKey;
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[j] = a.part[wave * 64 + j * kFinThreads + lane];
@@ -607,65 +609,70 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(FinalizeArgs a) {
         x[j] = wave * 64 + j * kFinThreads + lane < n_part && x[j] <= gb ? x[j] : kEmptyKey;
         least = x[j] < least ? x[j] : least;
     }
-    auto load_more = [&](int base, uint64_t (&y)[8]) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int i = base + j * kFinThreads + lane;
-            y[j] = i < n_part ? a.part[i] : kEmptyKey;
-            y[j] = y[j] <= gb ? y[j] : kEmptyKey;
-        }
-    };
-    for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
-        uint64_t y[8];
-        load_more(base, y);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) least = y[j] < least ? y[j] : least;
-    }
-    sh.lists[wave][lane] = least;
-    if (tid == 0) sh.s_misc[4] = 0;
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int w = 1; w < kFinWaves; ++w) least = sh.lists[w][lane] < least ? sh.lists[w][lane] : least;
-        const uint64_t kth = __shfl(wave_sort64(least, lane), k - 1);
-        if (lane == 0) sh.bound = kth;
-    }
-    __syncthreads();
-    const uint64_t cut = sh.bound;
-    uint64_t* const buf = sh.u.sort.key;                 // kSortCap keys
-    auto gather = [&](const uint64_t (&y)[8]) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (y[j] <= cut && y[j] != kEmptyKey) {
-                const int at = atomicAdd(&sh.s_misc[4], 1);
-                if (at < kFinThreads) buf[at] = y[j];
-            }
-        }
-    };
-    gather(x);
-    for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
-        uint64_t y[8];
-        load_more(base, y);
-        gather(y);
-    }
-    __syncthreads();
-    const int n_cut = sh.s_misc[4];
-    if (n_cut <= kFinThreads) {
-        if (wave * 64 < n_cut) {
-            list = wave_sort64(tid < n_cut ? buf[tid] : kEmptyKey, lane);
-            if (lane >= k) list = kEmptyKey;
-        }
-        list = tree_merge(sh, list, k, (n_cut + 63) / 64);
+    if (n_part <= kFinThreads) {
+        wave_offer(list, thr, x[0], lane, k);
+        list = tree_merge(sh, list, k, (n_part + 63) / 64);
     } else {
+        auto load_more = [&](int base, uint64_t (&y)[8]) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) wave_offer(list, thr, x[j] <= cut ? x[j] : kEmptyKey, lane, k);
+            for (int j = 0; j < 8; ++j) {
+                const int i = base + j * kFinThreads + lane;
+                y[j] = i < n_part ? a.part[i] : kEmptyKey;
+                y[j] = y[j] <= gb ? y[j] : kEmptyKey;
+            }
+        };
         for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
             uint64_t y[8];
             load_more(base, y);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) wave_offer(list, thr, y[j] <= cut ? y[j] : kEmptyKey, lane, k);
+            for (int j = 0; j < 8; ++j) least = y[j] < least ? y[j] : least;
         }
-        list = tree_merge(sh, list, k);
+        sh.lists[wave][lane] = least;
+        if (tid == 0) sh.s_misc[4] = 0;
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int w = 1; w < kFinWaves; ++w) least = sh.lists[w][lane] < least ? sh.lists[w][lane] : least;
+            const uint64_t kth = __shfl(wave_sort64(least, lane), k - 1);
+            if (lane == 0) sh.bound = kth;
+        }
+        __syncthreads();
+        const uint64_t cut = sh.bound;
+        uint64_t* const buf = sh.u.sort.key;                 // kSortCap keys
+        auto gather = [&](const uint64_t (&y)[8]) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (y[j] <= cut && y[j] != kEmptyKey) {
+                    const int at = atomicAdd(&sh.s_misc[4], 1);
+                    if (at < kFinThreads) buf[at] = y[j];
+                }
+            }
+        };
+        gather(x);
+        for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
+            uint64_t y[8];
+            load_more(base, y);
+            gather(y);
+        }
+        __syncthreads();
+        const int n_cut = sh.s_misc[4];
+        if (n_cut <= kFinThreads) {
+            if (wave * 64 < n_cut) {
+                list = wave_sort64(tid < n_cut ? buf[tid] : kEmptyKey, lane);
+                if (lane >= k) list = kEmptyKey;
+            }
+            list = tree_merge(sh, list, k, (n_cut + 63) / 64);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) wave_offer(list, thr, x[j] <= cut ? x[j] : kEmptyKey, lane, k);
+            for (int base = kFinThreads * 8 + wave * 64; base < n_part; base += kFinThreads * 8) {
+                uint64_t y[8];
+                load_more(base, y);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) wave_offer(list, thr, y[j] <= cut ? y[j] : kEmptyKey, lane, k);
+            }
+            list = tree_merge(sh, list, k);
+        }
     }
     if (wave == 0) {
         const int ns = __popcll(__ballot(lane < k && list != kEmptyKey));

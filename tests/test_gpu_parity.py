@@ -511,3 +511,26 @@ def test_seed_merge_with_ties_and_many_keys(k, copies, rng):
     if copies:
         same = np.flatnonzero(np.all(emb == emb[0], axis=1))
         np.testing.assert_array_equal(idx[: min(k, len(same))], same[: min(k, len(same))])
+
+
+# up to one key per thread (1,024) each wave sorts its own; more go through the cut
+@pytest.mark.parametrize("n", [3, 63, 200, 1500, 30_000])
+@pytest.mark.parametrize("k", [1, 2, 3, 16, 64])
+def test_seed_merge_of_few_keys(n, k, rng):
+    """The finalize kernel's merge of few keys: the seeds are the k best rows by (score, id)."""
+    emb, mods, ts, row, col, _ = random_graph(rng, n, 256)
+    ts[:] = 100.0
+    emb[n // 2] = emb[0]
+    dev = Dev(emb, mods, ts, row, col)
+    try:
+        mars_amd.query_memory_fast(dev.dg, dev.ctx, emb[0], T_Q, RetrievalConfig(
+            top_k=k, bfs_max_hops=0, time_decay_lambda=0.0, max_results_returned=k))
+        idx, val = dev.ctx.last_seeds()
+    finally:
+        dev.close()
+    dots = emb.astype(np.float64) @ emb[0].astype(np.float64)
+    m = min(n, k)
+    assert len(idx) == m and len(set(idx.tolist())) == m
+    assert np.all(dots[idx] >= np.sort(dots)[-m] - 1e-5) and np.all(np.abs(val - dots[idx]) <= 1e-5)
+    pair = list(zip((-val).tolist(), idx.tolist()))
+    assert pair == sorted(pair)
