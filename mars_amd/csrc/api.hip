@@ -628,15 +628,15 @@ int32_t mm_chunk(int64_t q, int64_t n) {
 }
 
 int64_t batch_part_room(int64_t held, int64_t need) {
-    return std::max(need, std::min(2 * held, kRqAllKeys));
+    return std::max(need, std::min(2 * held, kRqScoreWords));
 }
 
 // Row ranges x query blocks for the batched scan: one 512-thread workgroup per CU
 // (256 CUs), all query blocks of a row range on one XCD.
-void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
-                int32_t max_ranges, int32_t kp, bool rq64) {
+BatchGrid batch_grid(int64_t n, int32_t q, bool plain, int32_t kp, int32_t max_ranges, bool rq64) {
     // n_qblocks counts 64-query blocks (the layout of the partial keys) for every kernel
-    const int32_t qblocks = (q + 63) / 64;
+    BatchGrid b{};
+    b.n_qblocks = (q + 63) / 64;
     const bool gemm = batch_uses_gemm(q, plain), rq = batch_uses_rq(q, plain, rq64);
     const int32_t wgq = gemm ? 256 : (rq ? 64 * batch_rq_tiles(q) : 64);   // queries per workgroup
     const int32_t tiles = (q + wgq - 1) / wgq;                             // workgroups per row range
@@ -646,12 +646,16 @@ void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n
     if (gemm) rr = mm_ranges(tiles, max_rr);
     if (rr > max_ranges) rr = std::max(1, max_ranges);
     if (rr > max_rr) rr = int32_t(max_rr);
-    *n_qblocks = qblocks;
-    *rows_per_range = ((n + rr - 1) / rr + align - 1) / align * align;
-    if (rq && kp > 0 && *rows_per_range < kRqFloorTiles * align &&
-        int64_t(qblocks) * 64 * ((n + kp - 1) / kp * kp) <= kRqAllKeys)
-        *rows_per_range = kp;
-    *n_rranges = int32_t((n + *rows_per_range - 1) / *rows_per_range);
+    b.rows_per_range = ((n + rr - 1) / rr + align - 1) / align * align;
+    const int64_t score_words = int64_t(b.n_qblocks) * 64 * max_rr * align / 2;
+    if (rq && b.rows_per_range < kRqFloorTiles * align && score_words <= kRqScoreWords &&
+        (max_ranges >= 256 || max_rr <= max_ranges)) {
+        b.scores = 1;
+        b.rows_per_range = align;
+    }
+    b.n_rranges = int32_t((n + b.rows_per_range - 1) / b.rows_per_range);
+    b.part = b.scores ? score_words : int64_t(b.n_qblocks) * b.n_rranges * 64 * kp;
+    return b;
 }
 
 namespace {
@@ -1557,13 +1561,10 @@ int mars_query_batch(const mars_graph* gh, mars_ctx* ch, const float* dq, int32_
     MARS_TRY(use_device(c.device));
     const int32_t K = cfg->top_k;
     const int32_t n_live = __atomic_load_n(&g.n, __ATOMIC_ACQUIRE);
-    int32_t nrr = 0, nqb = 0;
-    int64_t rpr = 0;
-    const int32_t kp = batch_kpart(K);
     const bool uniform = std::all_of(h_tq, h_tq + Q, [&](float x) { return x == h_tq[0]; });
     const bool rq64 = batch_small_rq(Q, n_live, uniform);
-    batch_grid(n_live, Q, false, &nrr, &nqb, &rpr, 256, kp, rq64);
-    MARS_TRY(ensure_batch_scratch(c, Q, int64_t(nqb) * nrr * 64 * kp));
+    const BatchGrid bg = batch_grid(n_live, Q, false, batch_kpart(K), 256, rq64);
+    MARS_TRY(ensure_batch_scratch(c, Q, bg.part));
     hipStream_t s = c.stream;
     MARS_HIP(hipMemcpyAsync(c.btq, h_tq, size_t(Q) * sizeof(float), hipMemcpyHostToDevice, s));
     MARS_TRY(launch_f32_to_f16_rows(dq, c.bq, int64_t(Q) * g.d, s));
@@ -1572,7 +1573,8 @@ int mars_query_batch(const mars_graph* gh, mars_ctx* ch, const float* dq, int32_
     BatchArgs a{};
     a.emb16 = g.emb16; a.n = n_live; a.d = g.d; a.qh = c.bq; a.q = Q; a.tq = c.btq; a.ts = g.ts; a.mods = g.mods;
     a.lambda = cfg->time_decay_lambda; a.mod_filter = cfg->modality_filter; a.k = K; a.q_plain = Q; a.self_base = -1;
-    a.part = c.bpart; a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
+    a.part = c.bpart;
+    batch_layout(a, bg);
     a.uniform_tq = uniform ? 1 : 0;
     a.rq64 = rq64 ? 1 : 0;
     MARS_TRY(launch_batch_topk(a, K, c.bout, s, timing ? c.ev[1] : nullptr));
@@ -1747,13 +1749,9 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
             if (timing) MARS_HIP(hipEventRecord(c.ev[2], s));
             seed_stride = 64;
         } else {
-            int32_t nrr = 0, nqb = 0;
-            int64_t rpr = 0;
-            const int32_t kp = batch_kpart(kMultiCand);
-            const bool uniform = Qg == 0 || std::all_of(h_tq, h_tq + Qg, [&](float x) { return x == h_tq[0]; });
             const bool rq64 = batch_small_rq(Qt, n_live, uniform);
-            batch_grid(n_live, Qt, Qg == 0, &nrr, &nqb, &rpr, 256, kp, rq64);   // the k-NN queries alone: plain
-            MARS_TRY(ensure_batch_scratch(c, Qt, int64_t(nqb) * nrr * 64 * kp));
+            const BatchGrid bg = batch_grid(n_live, Qt, Qg == 0, batch_kpart(kMultiCand), 256, rq64);   // the k-NN queries alone: plain
+            MARS_TRY(ensure_batch_scratch(c, Qt, bg.part));
             if (Qg > 0) {
                 MARS_HIP(hipMemcpyAsync(c.btq, h_tq, size_t(Qg) * sizeof(float), hipMemcpyHostToDevice, s));
                 MARS_TRY(launch_f32_to_f16_rows(dq, c.bq, int64_t(Qg) * g.d, s));
@@ -1767,7 +1765,7 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
             b.emb16 = g.emb16; b.n = n_live; b.d = g.d; b.qh = c.bq; b.q = Qt; b.tq = c.btq; b.ts = g.ts;
             b.mods = g.mods; b.lambda = Qg > 0 ? lambda : 0.0f; b.mod_filter = Qg > 0 ? cfg->modality_filter : -1;
             b.k = kMultiCand; b.nrm = g.nrm; b.q_plain = Qg; b.self_base = knn_count > 0 ? knn_first : -1; b.part = c.bpart;
-            b.rows_per_range = rpr; b.n_rranges = nrr; b.n_qblocks = nqb;
+            batch_layout(b, bg);
             b.uniform_tq = uniform ? 1 : 0;
             b.rq64 = rq64 ? 1 : 0;
             MARS_TRY(launch_batch_topk(b, kMultiCand, c.bout, s));
@@ -2008,21 +2006,18 @@ int knn_lists(Graph& g, int32_t k, int64_t lo, int64_t hi, int64_t block, int32_
     constexpr int32_t kCand = 16;
     const int64_t n = g.n, count = hi - lo, most = block ? std::min(block, count) : count;
     const int32_t chunk = mm_chunk(block ? block : count, block ? block : n);   // queries per launch
-    int32_t nrr = 0, nqb = 0;
-    int64_t rpr = 0;
-    int64_t part_keys = 0;                           // the largest launch's
+    int64_t part_words = 0;                          // the largest launch's
     for (const int64_t nb : {most, block ? count % block : 0}) {
         for (const int64_t q : {std::min<int64_t>(chunk, nb), nb % chunk}) {
             if (q == 0) continue;
-            batch_grid(block ? nb : n, int32_t(q), true, &nrr, &nqb, &rpr, 256, kCand);
-            part_keys = std::max(part_keys, int64_t(nqb) * nrr * 64 * kCand);
+            part_words = std::max(part_words, batch_grid(block ? nb : n, int32_t(q), true, kCand).part);
         }
     }
     const auto pad = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
     const size_t n_dn = size_t(count) * k * sizeof(int32_t), n_cert = size_t(count) * sizeof(int32_t);
     const size_t o_dn = 0, o_cert = pad(n_dn), o_tq = o_cert + pad(n_cert), o_cand = o_tq + pad(size_t(chunk) * sizeof(float)),
                  o_part = o_cand + pad(size_t(chunk) * kCand * sizeof(uint64_t)),
-                 bytes = o_part + size_t(part_keys) * sizeof(uint64_t);
+                 bytes = o_part + size_t(part_words) * sizeof(uint64_t);
     MARS_TRY(knn_workspace(g, bytes, o_cert + n_cert));
     unsigned char* const ws = static_cast<unsigned char*>(g.knn_ws);
     int32_t* const dn = reinterpret_cast<int32_t*>(ws + o_dn);
@@ -2039,12 +2034,11 @@ int knn_lists(Graph& g, int32_t k, int64_t lo, int64_t hi, int64_t block, int32_
         const int64_t r0 = block ? b0 : 0, rows = block ? std::min(block, n - b0) : n, q1 = block ? b0 + rows : hi;
         for (int64_t q0 = b0; q0 < q1 && rc == MARS_OK; q0 += chunk) {
             const int32_t q = int32_t(std::min<int64_t>(chunk, q1 - q0));
-            batch_grid(rows, q, true, &nrr, &nqb, &rpr, 256, kCand);
             BatchArgs a{};
             a.emb16 = g.emb16 + r0 * g.d; a.n = rows; a.d = g.d; a.qh = g.emb16 + q0 * g.d; a.q = q; a.tq = tq;
             a.ts = g.ts + r0; a.mods = g.mods + r0; a.lambda = 0.0f; a.mod_filter = -1; a.k = kCand; a.nrm = g.nrm;
             a.q_plain = 0; a.self_base = q0 - r0; a.part = part; a.uniform_tq = 1;
-            a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
+            batch_layout(a, batch_grid(rows, q, true, kCand));
             rc = launch_batch_topk(a, kCand, cand, s);
             if (rc == MARS_OK)
                 rc = launch_knn_rerank(g.emb + r0 * g.d, q0 - r0, q, g.d, cand, kCand, k, dn + (q0 - lo) * k, s, g.nrm,

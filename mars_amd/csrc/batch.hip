@@ -236,10 +236,13 @@ __global__ __launch_bounds__(kBWaves * 64) void k_batch_scan(BatchArgs a) {
 constexpr int kMergeWaves = 8;
 constexpr int kMergeLd = 8;
 constexpr int kRerankPieces = 3;  // k_knn_rerank: 16-byte pieces per lane and row (d <= 768)
-template <int W>
+// SCORES: n_rranges tiles of 16 scores instead (BatchArgs::scores), rows past n_rows and the query's own row
+// left out here.
+template <int W, bool SCORES>
 __global__ __launch_bounds__(W == 1 ? 256 : W * 64) void k_batch_merge(const uint64_t* __restrict__ part,
                                                                       int32_t n_rranges, int32_t kpart, int32_t q,
-                                                                      int32_t k_out, uint64_t* __restrict__ out) {
+                                                                      int32_t k_out, uint64_t* __restrict__ out,
+                                                                      int32_t n_rows, int64_t self_base, int32_t q_plain) {
     __shared__ uint64_t s_l[W == 1 ? 4 : W][64];
     __shared__ uint64_t s_best[W == 1 ? 4 : 1][64];
     __shared__ uint32_t s_n;
@@ -249,16 +252,23 @@ __global__ __launch_bounds__(W == 1 ? 256 : W * 64) void k_batch_merge(const uin
     if (qi >= q) return;                               // the whole workgroup, or (W = 1) the wave
     const int qb = qi / kBQ, j = qi % kBQ;
     const int total = n_rranges * kpart;
-    const int kshift = kpart == 8 ? 3 : 4;             // kpart is 8 or 16 (batch_kpart)
+    const int kshift = SCORES || kpart == 16 ? 4 : 3;  // kpart is 8 or 16 (batch_kpart)
+    const int32_t own = SCORES && self_base >= 0 && qi >= q_plain ? int32_t(self_base + (qi - q_plain)) : -1;
     const auto load = [&](int base, uint64_t (&xs)[kMergeLd]) {
 #pragma unroll
         for (int c = 0; c < kMergeLd; ++c) {
             const int t = base + c * 64 + lane;
             const bool on = t < total;                 // (total is a multiple of kpart: whole lists)
             const int list = on ? t >> kshift : 0;
-            const uint64_t x =
-                part[((int64_t(qb) * n_rranges + list) * kBQ + j) * kpart + ((t + (t >> 6)) & (kpart - 1))];
-            xs[c] = on ? x : kEmptyKey;
+            const int slot = (t + (t >> 6)) & ((1 << kshift) - 1);
+            const int64_t at = (((int64_t(qb) * n_rranges + list) * kBQ + j) << kshift) + slot;
+            if constexpr (SCORES) {
+                const int32_t row = list * 16 + slot;
+                const uint64_t x = make_key(reinterpret_cast<const float*>(part)[at], uint32_t(row));
+                xs[c] = on && row < n_rows && row != own ? x : kEmptyKey;
+            } else {
+                xs[c] = on ? part[at] : kEmptyKey;
+            }
         }
     };
     // the first round's keys stay in registers; later rounds' (many ranges) are read again
@@ -470,30 +480,31 @@ bool batch_uses_rq(int32_t q, bool plain, bool rq64) {
 bool batch_small_rq(int32_t q, int64_t n, bool uniform) {
     return q <= kRqMaxScanQ && (uniform || n <= (kRqFloorTiles - 1) * 16 * 256);
 }
-bool batch_keeps_all(const BatchArgs& a, int32_t kp) {
-    return batch_uses_rq(a.q, a.q_plain == 0, a.rq64 != 0) && a.rows_per_range == kp;
-}
 int batch_rq_tiles(int32_t q) { return q <= 64 ? 1 : q <= 128 ? 2 : 4; }
 int batch_kpart(int32_t k) { return k <= 8 ? 8 : 16; }
 
 int launch_batch_scan(const BatchArgs& a, hipStream_t s) {
     MARS_CHECK(a.k >= 1 && a.k <= 16, MARS_ERR_UNSUPPORTED, "batched scoring keeps at most 16 per query (asked %d)",
                a.k);
-    return a.k <= 8 ? launch_batch_k<8>(a, s) : launch_batch_k<16>(a, s);
-}
-
-int launch_batch_merge(const uint64_t* part, int32_t n_rranges, int32_t kpart, int32_t q, int32_t k_out,
-                       uint64_t* out, hipStream_t s) {
-    MARS_CHECK(kpart == 8 || kpart == 16, MARS_ERR_INVALID, "batched merge: %d keys per range", kpart);
-    if (n_rranges * kpart <= 64 * kMergeLd)
-        MARS_LAUNCH((k_batch_merge<1>), dim3(unsigned((q + 3) / 4)), dim3(256), 0, s, part, n_rranges, kpart, q, k_out, out);
-    else
-        MARS_LAUNCH((k_batch_merge<kMergeWaves>), dim3(unsigned(q)), dim3(kMergeWaves * 64), 0, s, part, n_rranges, kpart,
-                    q, k_out, out);
-    return MARS_OK;
+    return a.k <= 8 && !a.scores ? launch_batch_k<8>(a, s) : launch_batch_k<16>(a, s);
 }
 
 namespace {
+
+template <bool SCORES>
+int launch_merge_t(const BatchArgs& a, int32_t kp, int32_t k_out, uint64_t* out, hipStream_t s) {
+    if (a.n_rranges * kp <= 64 * kMergeLd)
+        MARS_LAUNCH((k_batch_merge<1, SCORES>), dim3(unsigned((a.q + 3) / 4)), dim3(256), 0, s, a.part, a.n_rranges, kp, a.q,
+                    k_out, out, int32_t(a.n), a.self_base, a.q_plain);
+    else
+        MARS_LAUNCH((k_batch_merge<kMergeWaves, SCORES>), dim3(unsigned(a.q)), dim3(kMergeWaves * 64), 0, s, a.part,
+                    a.n_rranges, kp, a.q, k_out, out, int32_t(a.n), a.self_base, a.q_plain);
+    return MARS_OK;
+}
+
+int launch_batch_merge(const BatchArgs& a, int32_t k_out, uint64_t* out, hipStream_t s) {
+    return a.scores ? launch_merge_t<true>(a, 16, k_out, out, s) : launch_merge_t<false>(a, batch_kpart(a.k), k_out, out, s);
+}
 
 // The rows of each range that k_batch_rq's sampled pass covers (0: no sampled pass). A pass over s
 // of a range's T tiles costs s tiles; without it a query meets about kp T / s rows per range and
@@ -520,8 +531,10 @@ int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, 
     // Without a floor a query inserts about K (1 + ln(rows / K)) rows per range (every new best of
     // the rows seen so far), with it about rows x K / sampled rows.
     const bool gemm = batch_uses_gemm(a.q, a.q_plain == 0);
-    a.sample_pass = batch_keeps_all(a, kp) ? 1 : 0;   // one pass, every row's key
-    const int64_t rq_rows = batch_uses_rq(a.q, a.q_plain == 0, a.rq64 != 0) ? rq_sample_rows(a, kp) : 0;
+    a.sample_pass = 0;
+    const bool rq = batch_uses_rq(a.q, a.q_plain == 0, a.rq64 != 0);
+    MARS_CHECK(!a.scores || rq, MARS_ERR_INVALID, "batched scoring: %d queries keep lists", a.q);
+    const int64_t rq_rows = rq && !a.scores ? rq_sample_rows(a, kp) : 0;
     if (gemm || rq_rows > 0) {
         BatchArgs b = a;
         b.rows_per_range = gemm ? std::min<int64_t>(a.rows_per_range, (kMmSampleTiles + a.n_rranges - 1) / a.n_rranges * 256)
@@ -529,13 +542,13 @@ int launch_batch_topk(BatchArgs a, int32_t k_out, uint64_t* out, hipStream_t s, 
         b.range_stride = a.rows_per_range;
         b.sample_pass = 1;
         MARS_TRY(launch_batch_scan(b, s));
-        MARS_TRY(launch_batch_merge(a.part, a.n_rranges, kp, a.q, k_out, out, s));
+        MARS_TRY(launch_batch_merge(a, k_out, out, s));
         a.floor_keys = out;
         a.floor_k = k_out;
     }
     MARS_TRY(launch_batch_scan(a, s));
     if (scanned != nullptr) MARS_HIP(hipEventRecord(scanned, s));
-    return launch_batch_merge(a.part, a.n_rranges, kp, a.q, k_out, out, s);
+    return launch_batch_merge(a, k_out, out, s);
 }
 
 int launch_knn_rerank(const float* emb, int64_t q0, int64_t nq, int32_t d, const uint64_t* cand, int32_t kc,

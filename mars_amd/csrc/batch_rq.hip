@@ -83,7 +83,7 @@ __device__ __attribute__((always_inline)) inline void dma4(const void* g, uint32
     __builtin_amdgcn_global_load_lds(g, lds, 4, 0, 0);
 }
 
-// Workgroups per query group of a launch that keeps every row: one tile each, at most 256 in all.
+// Workgroups per query group of a launch that keeps every row's score: one tile each, at most 256 in all.
 __host__ __device__ inline int rq_all_wgs(const BatchArgs& a) {
     const int wgq = a.q <= 64 ? 64 : a.q <= 128 ? 128 : 256, groups = (a.q + wgq - 1) / wgq;
     const int64_t tiles = (a.n + kRRows - 1) / kRRows, most = 256 / groups > 1 ? 256 / groups : 1;
@@ -92,7 +92,7 @@ __host__ __device__ inline int rq_all_wgs(const BatchArgs& a) {
 
 // QT: 16-query MFMA tiles per wave (1, 2 or 4: 64, 128 or 256 queries per workgroup). MODE: the
 // full pass keeps the best K keys per query and range; the sampled pass of launch_batch_topk
-// keeps K row-class maxima instead; kRqAll writes every row's key (batch_keeps_all).
+// keeps K row-class maxima instead; kRqAll writes every row's score (BatchArgs::scores).
 constexpr int kRqFull = 0, kRqSample = 1, kRqAll = 2;
 template <int NS, int K, int QT, int MODE>
 __global__ __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -108,7 +108,7 @@ void k_batch_rq(BatchArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = lane & 15, kg = lane >> 4;
     constexpr int d = NS * 32;
-    // every row's key (batch_keeps_all): the tiles are dealt out evenly, wg_rows per workgroup
+    // every row's score: the tiles are dealt out evenly, wg_rows per workgroup
     const int n_wg = ALL ? rq_all_wgs(a) : a.n_rranges;           // workgroups per query group
     const int wg_rows = int((a.n + kRRows * n_wg - 1) / (kRRows * n_wg)) * kRRows;
     const int r_id = int(blockIdx.x) % n_wg;
@@ -495,11 +495,11 @@ void k_batch_rq(BatchArgs a) {
                         if constexpr (!ALL) {
                             mx[4 * qt + v] = in ? fmaxf(mx[4 * qt + v], sv) : mx[4 * qt + v];
                         } else {
-                            // row t0 + m is key (t0 + m) % K of range (t0 + m) / K
-                            const int q = qi + a.q_plain, row = t0 + m;
-                            if (q < a.q && row / K < a.n_rranges)
-                                a.part[((int64_t(q / 64) * a.n_rranges + row / K) * 64 + q % 64) * K + row % K] =
-                                    in ? make_key(sv, uint32_t(row)) : kEmptyKey;
+                            // row t0 + m is score m of range (t0 + m) / 16 (the query's own row among
+                            // them; rows past the last are not written)
+                            const int q = qi + a.q_plain;
+                            if (q < a.q && m < nr)
+                                reinterpret_cast<float*>(a.part)[((int64_t(q / 64) * a.n_rranges + t0 / kRRows) * 64 + q % 64) * kRRows + m] = sv;
                         }
                     }
                 }
@@ -545,11 +545,14 @@ void k_batch_rq(BatchArgs a) {
 template <int NS, int K, int QT>
 int launch_rq_q(const BatchArgs& a, hipStream_t s) {
     constexpr int wgq = kRWaves * 16 * QT;       // queries per workgroup
-    const bool all = a.sample_pass && a.range_stride == 0;
-    const unsigned grid = unsigned((all ? rq_all_wgs(a) : a.n_rranges) * ((a.q + wgq - 1) / wgq));
-    if (all)
-        MARS_LAUNCH((k_batch_rq<NS, K, QT, kRqAll>), dim3(grid), dim3(kRThreads), 0, s, a);
-    else if (a.sample_pass)
+    const unsigned grid = unsigned((a.scores ? rq_all_wgs(a) : a.n_rranges) * ((a.q + wgq - 1) / wgq));
+    if constexpr (K == 16) {
+        if (a.scores) {
+            MARS_LAUNCH((k_batch_rq<NS, K, QT, kRqAll>), dim3(grid), dim3(kRThreads), 0, s, a);
+            return MARS_OK;
+        }
+    }
+    if (a.sample_pass)
         MARS_LAUNCH((k_batch_rq<NS, K, QT, kRqSample>), dim3(grid), dim3(kRThreads), 0, s, a);
     else
         MARS_LAUNCH((k_batch_rq<NS, K, QT, kRqFull>), dim3(grid), dim3(kRThreads), 0, s, a);
@@ -584,7 +587,7 @@ int launch_batch_rq(const BatchArgs& a, hipStream_t s) {
     MARS_CHECK(a.n <= INT32_MAX - 64, MARS_ERR_CAPACITY, "batched scoring: %lld rows", (long long)a.n);
     MARS_CHECK(a.n_qblocks == (a.q + 63) / 64, MARS_ERR_INVALID, "batched scoring: %d query blocks for %d queries",
                a.n_qblocks, a.q);
-    return a.k <= 8 ? launch_rq_k<8>(a, s) : launch_rq_k<16>(a, s);
+    return a.k <= 8 && !a.scores ? launch_rq_k<8>(a, s) : launch_rq_k<16>(a, s);
 }
 
 }  // namespace mars

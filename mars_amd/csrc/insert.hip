@@ -55,8 +55,8 @@ constexpr int32_t kKnnCand = 16;            // fp16 candidates rescored per new 
 // search's duration, so it applies up to kInsertKnnNarrowRows rows: beyond them one
 // search per insert call already fills a large share of the GPU (at 13M rows a
 // full-width search takes about 4 ms), and a longer one would only delay the writer.
-// (Every range keeps lists: a layout that keeps each row's key has more ranges than these, and
-// grew its buffer with the graph, 900 nodes inserted into 6,300 rows 142 -> 410 us.)
+// (The layout that keeps every row's score has a range per 16 rows, so it serves up to 1,024 rows here;
+// without the cap its buffer grew with the graph, 900 nodes inserted into 6,300 rows 142 -> 410 us.)
 constexpr int32_t kInsertKnnRanges = 64;
 constexpr int64_t kInsertKnnNarrowRows = 2000000;
 // Up to that size the narrow fp16 search runs first, its lists certified as the k-NN
@@ -284,8 +284,8 @@ int insert_knn_int8(Graph& g, int64_t first, int32_t nq, int64_t n, int32_t k, h
 
 }  // namespace
 
-void insert_grid(int64_t n, int32_t q, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range) {
-    batch_grid(n, q, true, n_rranges, n_qblocks, rows_per_range, n <= kInsertKnnNarrowRows ? kInsertKnnRanges : 256);
+BatchGrid insert_grid(int64_t n, int32_t q) {
+    return batch_grid(n, q, true, kKnnCand, n <= kInsertKnnNarrowRows ? kInsertKnnRanges : 256);
 }
 
 namespace {
@@ -295,12 +295,10 @@ namespace {
 // first + i's list is certified exact (its k-th exact score beats the 16th candidate's
 // fp16 score by the fp16 error bound).
 int insert_knn_fp16(Graph& g, int64_t first, int32_t nq, int64_t n, int32_t k, hipStream_t s, int32_t* cert) {
-    int32_t nrr = 0, nqb = 0;
-    int64_t rpr = 0, part_keys = 0;
+    int64_t part_keys = 0;
     for (int32_t q : {std::min(nq, kInsertChunk), nq % kInsertChunk}) {   // full and last chunk
         if (q == 0) continue;
-        insert_grid(n, q, &nrr, &nqb, &rpr);
-        part_keys = std::max<int64_t>(part_keys, int64_t(nrr) * nqb * 64 * kKnnCand);
+        part_keys = std::max(part_keys, insert_grid(n, q).part);
     }
     if (part_keys > g.ins_part_cap) {
         dfree(g.ins_part);
@@ -321,12 +319,12 @@ int insert_knn_fp16(Graph& g, int64_t first, int32_t nq, int64_t n, int32_t k, h
     }
     for (int32_t c0 = 0; c0 < nq; c0 += kInsertChunk) {
         const int32_t q = std::min(kInsertChunk, nq - c0);
-        insert_grid(n, q, &nrr, &nqb, &rpr);
         BatchArgs a{};
         a.emb16 = g.emb16; a.n = n; a.d = g.d; a.qh = g.emb16 + (first + c0) * g.d; a.q = q; a.tq = g.ins_tq;
         a.ts = g.ts; a.mods = g.mods; a.lambda = 0.0f; a.mod_filter = -1; a.k = kKnnCand;
-        a.nrm = g.nrm; a.q_plain = 0; a.self_base = first + c0; a.part = g.ins_part; a.rows_per_range = rpr; a.n_rranges = nrr;
-        a.n_qblocks = nqb; a.uniform_tq = 1;
+        a.nrm = g.nrm; a.q_plain = 0; a.self_base = first + c0; a.part = g.ins_part;
+        batch_layout(a, insert_grid(n, q));
+        a.uniform_tq = 1;
         MARS_TRY(launch_batch_topk(a, kKnnCand, g.ins_cand, s));
         MARS_TRY(launch_knn_rerank(g.emb, first + c0, q, g.d, g.ins_cand, kKnnCand, k, g.ins_nbrs + int64_t(c0) * k, s,
                                    cert ? g.nrm : nullptr, cert ? cert + c0 : nullptr));

@@ -83,20 +83,25 @@ void dfree(T*& p) {
     p = nullptr;
 }
 
-// Row ranges x query blocks of the batched scan (defined in api.hip). plain: every query
-// is a neighbour search (BatchArgs::q_plain == 0), which picks the kernel as in
-// batch_uses_gemm. max_ranges caps the row ranges (workgroups per 64-query block). kp (without a
-// cap): the keys per query and range the launch keeps (batch_kpart), or 0; with it a k_batch_rq launch of few
-// rows gets ranges of kp rows, which keep every row (batch_keeps_all), while their keys number at most
-// kRqAllKeys.
-void batch_grid(int64_t n, int32_t q, bool plain, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range,
-                int32_t max_ranges = 256, int32_t kp = 0, bool rq64 = false);
-// The keys a scratch that held `held` of them and must hold `need` is given: twice as many as before,
-// up to kRqAllKeys. (With every row's key kept, need follows the row count of a growing graph: exact
-// sizes would be allocated again, and the device waited for, every few inserts.)
+// Row ranges x query blocks of a batched launch (batch_grid, api.hip).
+struct BatchGrid {
+    int32_t n_rranges;
+    int32_t n_qblocks;       // of 64 queries
+    int64_t rows_per_range;
+    int64_t part;            // 64-bit words of BatchArgs::part
+    int32_t scores;          // BatchArgs::scores
+};
+// plain: every query is a neighbour search (BatchArgs::q_plain == 0), which picks the kernel as in
+// batch_uses_gemm. kp: the keys per query and range of its lists (batch_kpart). max_ranges caps the
+// row ranges (workgroups per 64-query block). A k_batch_rq launch of few rows keeps every row's score
+// instead, in ranges of one tile (BatchArgs::scores), where the cap allows so many.
+BatchGrid batch_grid(int64_t n, int32_t q, bool plain, int32_t kp, int32_t max_ranges = 256, bool rq64 = false);
+// The words of BatchArgs::part that a scratch which held `held` and must hold `need` is given: twice as
+// many as before, up to kRqScoreWords. (With every row's score kept, need follows the row count of a growing
+// graph: exact sizes would be allocated again, and the device waited for, every few inserts.)
 int64_t batch_part_room(int64_t held, int64_t need);
-// The same for an insert's neighbour search of q new nodes (insert.hip): few ranges, lists only.
-void insert_grid(int64_t n, int32_t q, int32_t* n_rranges, int32_t* n_qblocks, int64_t* rows_per_range);
+// The grid of an insert's neighbour search of q new nodes among n rows (insert.hip): few ranges.
+BatchGrid insert_grid(int64_t n, int32_t q);
 
 constexpr int kMaxK = 64;              // seeds per query (wave-held list), as MAX_TOP_K
 constexpr int kSortCap = 8192;         // results sorted in LDS by the finalize kernel (one band)
@@ -533,7 +538,7 @@ struct BatchArgs {
     int64_t self_base;       // >= 0: neighbour search j (query q_plain + j) is node self_base + j
                              // and never its own neighbour
     const uint32_t* nrm;     // optional (k_batch_mm): the fp16 copy's row-norm maxima
-    uint64_t* part;          // [n_qblocks][n_rranges][64][K] keys
+    uint64_t* part;          // [n_qblocks][n_rranges][64][K] keys, or (scores) [..][64][16] fp32 scores
     int64_t rows_per_range;
     int64_t range_stride;    // row range r starts at row r * range_stride (0: rows_per_range)
     const uint64_t* floor_keys;  // optional: query j keeps no row below the score of key
@@ -543,9 +548,17 @@ struct BatchArgs {
     int32_t n_qblocks;
     int32_t uniform_tq;      // all query times equal: one decay weight per row
     int32_t rq64;            // up to 64 queries: k_batch_rq, not k_batch_scan (batch_small_rq)
+    int32_t scores;          // k_batch_rq writes every row's score, a range per 16-row tile; rows past the
+                             // last and a search's own row are left to the merge
     int32_t sample_pass;     // the sampled pass of launch_batch_topk: its keys serve only as
                              // floors (k_batch_mm then keeps group maxima, not the best K)
 };
+inline void batch_layout(BatchArgs& a, const BatchGrid& g) {
+    a.rows_per_range = g.rows_per_range;
+    a.n_rranges = g.n_rranges;
+    a.n_qblocks = g.n_qblocks;
+    a.scores = g.scores;
+}
 bool batch_dim_supported(int32_t d);
 // Three kernels score a batch, by its size and kind (1M rows, d = 768, one MI355X):
 //   Q <= kRqMaxScanQ              k_batch_scan: 64-query blocks, rows streamed into registers
@@ -587,36 +600,34 @@ bool batch_uses_gemm(int32_t q, bool plain);
 // rq64: a batch of up to 64 queries may take k_batch_rq too (BatchArgs::rq64)
 bool batch_uses_rq(int32_t q, bool plain, bool rq64);
 // Whether a batch of up to 64 queries takes k_batch_rq (one 16-query tile per wave) rather than
-// k_batch_scan: with one query time, or where every row's key is kept. (The whole call, k_batch_scan
+// k_batch_scan: with one query time, or where every row's score is kept. (The whole call, k_batch_scan
 // / k_batch_rq: 64 queries over 1M rows of 768, one time 347 / 323 us, per-query times and decay
 // 374 / 392; 17 over 300K 139 / 137 and 142 / 166; 64 over 30,000 88 / 65 and 90 / 67; 1 over 6,000
 // 65 / 43 us. Inserts' neighbour searches stay with k_batch_scan, which leaves a CU's LDS to
 // the queries beside them.)
 bool batch_small_rq(int32_t q, int64_t n, bool uniform);
-// A k_batch_rq launch whose ranges hold as many rows as keys: its product is written whole, a
-// key per row, and the merge selects. batch_grid lays launches out so where a workgroup would have
-// fewer than kRqFloorTiles tiles: there a floor's passes (rq_sample_rows) and filling and searching
-// lists cost more than a longer merge. (The whole call, with lists and floor / so: 438 queries
-// over 6,307 rows, 4 tiles, 90 / 74 us; 512 over 12,000, 6 tiles, 117 / 90; 256 over 40,000, 10
-// tiles, 122 / 110; 100 over 50,000, 13 tiles, 98 / 98; 80 over 60,000, 15 tiles, 88 / 106 us.)
+// k_batch_rq keeps every row's score (BatchArgs::scores), and the merge selects, where a workgroup would
+// have fewer than kRqFloorTiles tiles: there a floor's passes (rq_sample_rows) and filling and searching
+// lists cost more than a longer merge. (The whole call over rows of 768, one time, lists and floor / scores,
+// 10 results, without decay and with: 600 queries over 12,000 rows, 10 tiles, 121 / 90 and 112 / 91 us; 200
+// over 38,000, 10 tiles, 106 / 91 and 96 / 93; 128 over 49,000, 12 tiles, 92 / 84 and 86 / 86; 65 over 65,000,
+// 16 tiles, 91 / 94 and 87 / 94. As 64-bit keys in ranges of the lists' length: 256 queries over 20,000 rows,
+// up to 8 results, 85 us, 72 as scores.)
 constexpr int64_t kRqFloorTiles = 12;
-// At most 48 MiB of keys (one per query and row; the lists' layout needs 32 KiB per query at most,
-// whatever the rows).
-constexpr int64_t kRqAllKeys = int64_t(6) << 20;
+// At most 48 MiB of scores: 512 queries over any rows that few tiles hold, and a larger batch's over
+// fewer (the lists' layout needs 32 KiB per query at most, whatever the rows).
+constexpr int64_t kRqScoreWords = int64_t(6) << 20;
 // Ranges of fewer tiles than this keep lists without a floor, whose pass over 1 tile of 2 or 3 costs
 // what it saves. (Lists of short ranges are k_batch_rq's slowest form: the whole call without / with a
 // floor, one query time: 256 queries over 40,000 rows, 10 tiles, 183 / 94 us; over 24,000, 6 tiles, 128 / 86;
 // 4 tiles 98 / 81; 3 tiles 83 / 77 and, over 8,000, 2 tiles, 69 / 77.)
 constexpr int64_t kRqListTiles = 4;
-bool batch_keeps_all(const BatchArgs& a, int32_t kp);
-int batch_rq_tiles(int32_t q);   // 16-query MFMA tiles per k_batch_rq wave: 2 or 4
+int batch_rq_tiles(int32_t q);   // 16-query MFMA tiles per k_batch_rq wave: 1, 2 or 4
 int launch_batch_rq(const BatchArgs& a, hipStream_t s);
 int batch_kpart(int32_t k);  // keys per (query, row range) the scan writes
 int launch_batch_scan(const BatchArgs& a, hipStream_t s);
 // Batches of at least kGemmMinQ queries: k_batch_mm (batch_mm.hip).
 int launch_batch_mm(const BatchArgs& a, hipStream_t s);
-int launch_batch_merge(const uint64_t* part, int32_t n_rranges, int32_t kpart, int32_t q, int32_t k_out,
-                       uint64_t* out, hipStream_t s);
 // Scoring plus the merge: out[j * k_out ..] = query j's k_out best keys over all rows. For more
 // than kRqMaxScanQ queries (k_batch_rq, k_batch_mm) a first pass over the first rows of every
 // range keeps maxima over classes of rows, merged into out: each query's k_out-th best is a floor

@@ -29,9 +29,9 @@ namespace {
 constexpr int32_t kStaticMaxQ = 256;                      // queries per call
 constexpr int32_t kStaticMaxD = 768;                      // widest batched row (batch_dim_supported)
 constexpr size_t kStaticQBytes = size_t(kStaticMaxQ) * kStaticMaxD * sizeof(__half);     // 384 KiB
-// 48 MiB of partial keys: every row's, wherever mars_query_batch keeps them. (With 8 MiB, which the
-// lists of any 256 queries fit, 256 queries over 12,000 rows took 83 us as lists, 55 us so.)
-constexpr size_t kStaticPartKeys = size_t(kRqAllKeys);
+// 48 MiB of partial keys, or of every row's score wherever mars_query_batch keeps them. (With 8 MiB, which
+// the lists of any 256 queries fit, 256 queries over 12,000 rows took 83 us as lists, 55 us so.)
+constexpr size_t kStaticPartKeys = size_t(kRqScoreWords);
 constexpr size_t kStaticOutKeys = size_t(kStaticMaxQ) * 16;
 constexpr size_t kStaticPartOff = (kStaticQBytes + 255) / 256 * 256;
 constexpr size_t kStaticOutOff = kStaticPartOff + kStaticPartKeys * sizeof(uint64_t);
@@ -102,13 +102,9 @@ extern "C" int mars_query_batch_static(const mars_graph* gh, const float* d_quer
     const int32_t K = cfg->top_k;
     const int32_t n_live = __atomic_load_n(&g.n, __ATOMIC_ACQUIRE);
     MARS_CHECK(n_live > 0, MARS_ERR_INVALID, "empty graph");
-    int32_t nrr = 0, nqb = 0;
-    int64_t rpr = 0;
-    const int32_t kp = batch_kpart(K);
-    batch_grid(n_live, Q, false, &nrr, &nqb, &rpr, 256, kp);
-    const int64_t part_keys = int64_t(nqb) * nrr * 64 * kp;
-    MARS_CHECK(part_keys <= int64_t(kStaticPartKeys), MARS_ERR_CAPACITY,
-               "mars_query_batch_static: %lld partial keys exceed the static %zu", (long long)part_keys,
+    const BatchGrid bg = batch_grid(n_live, Q, false, batch_kpart(K));
+    MARS_CHECK(bg.part <= int64_t(kStaticPartKeys), MARS_ERR_CAPACITY,
+               "mars_query_batch_static: %lld partial keys exceed the static %zu", (long long)bg.part,
                kStaticPartKeys);
     __half* bq = reinterpret_cast<__half*>(base);
     uint64_t* part = reinterpret_cast<uint64_t*>(base + kStaticPartOff);
@@ -118,7 +114,8 @@ extern "C" int mars_query_batch_static(const mars_graph* gh, const float* d_quer
     BatchArgs a{};
     a.emb16 = g.emb16; a.n = n_live; a.d = g.d; a.qh = bq; a.q = Q; a.tq = d_tq; a.ts = g.ts; a.mods = g.mods;
     a.lambda = cfg->time_decay_lambda; a.mod_filter = cfg->modality_filter; a.k = K; a.q_plain = Q; a.self_base = -1;
-    a.part = part; a.rows_per_range = rpr; a.n_rranges = nrr; a.n_qblocks = nqb;
+    a.part = part;
+    batch_layout(a, bg);
     a.uniform_tq = uniform_tq ? 1 : 0;
     MARS_TRY(launch_batch_topk(a, K, out, s));
     const int32_t n = Q * K;
