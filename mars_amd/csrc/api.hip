@@ -1562,7 +1562,7 @@ int mars_query_batch(const mars_graph* gh, mars_ctx* ch, const float* dq, int32_
     const int32_t K = cfg->top_k;
     const int32_t n_live = __atomic_load_n(&g.n, __ATOMIC_ACQUIRE);
     const bool uniform = std::all_of(h_tq, h_tq + Q, [&](float x) { return x == h_tq[0]; });
-    const bool rq64 = batch_small_rq(Q, n_live, uniform);
+    const bool rq64 = batch_small_rq(Q, n_live, g.d, K, uniform);
     const BatchGrid bg = batch_grid(n_live, Q, false, batch_kpart(K), 256, rq64);
     MARS_TRY(ensure_batch_scratch(c, Q, bg.part));
     hipStream_t s = c.stream;
@@ -1749,7 +1749,7 @@ int global_batch_impl(const mars_graph* gh, mars_ctx* ch, const float* dq, int32
             if (timing) MARS_HIP(hipEventRecord(c.ev[2], s));
             seed_stride = 64;
         } else {
-            const bool rq64 = batch_small_rq(Qt, n_live, uniform);
+            const bool rq64 = batch_small_rq(Qt, n_live, g.d, kMultiCand, uniform);
             const BatchGrid bg = batch_grid(n_live, Qt, Qg == 0, batch_kpart(kMultiCand), 256, rq64);   // the k-NN queries alone: plain
             MARS_TRY(ensure_batch_scratch(c, Qt, bg.part));
             if (Qg > 0) {

@@ -477,8 +477,10 @@ bool batch_uses_gemm(int32_t q, bool plain) { return plain && q >= kGemmMinQ; }
 bool batch_uses_rq(int32_t q, bool plain, bool rq64) {
     return (q > kRqMaxScanQ || rq64) && !batch_uses_gemm(q, plain);
 }
-bool batch_small_rq(int32_t q, int64_t n, bool uniform) {
-    return q <= kRqMaxScanQ && (uniform || n <= (kRqFloorTiles - 1) * 16 * 256);
+bool batch_small_rq(int32_t q, int64_t n, int32_t d, int32_t k, bool uniform) {
+    if (q > kRqMaxScanQ) return false;
+    if (n <= (k > 8 ? kRqFloorTiles - 1 : 8) * 16 * 256) return true;      // every row's score
+    return uniform && k > 8 && (d == 768 || n <= (d == 256 ? int64_t(1) << 19 : int64_t(1) << 20));
 }
 int batch_rq_tiles(int32_t q) { return q <= 64 ? 1 : q <= 128 ? 2 : 4; }
 int batch_kpart(int32_t k) { return k <= 8 ? 8 : 16; }

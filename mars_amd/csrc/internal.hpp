@@ -600,12 +600,15 @@ bool batch_uses_gemm(int32_t q, bool plain);
 // rq64: a batch of up to 64 queries may take k_batch_rq too (BatchArgs::rq64)
 bool batch_uses_rq(int32_t q, bool plain, bool rq64);
 // Whether a batch of up to 64 queries takes k_batch_rq (one 16-query tile per wave) rather than
-// k_batch_scan: with one query time, or where every row's score is kept. (The whole call, k_batch_scan
-// / k_batch_rq: 64 queries over 1M rows of 768, one time 347 / 323 us, per-query times and decay
-// 374 / 392; 17 over 300K 139 / 137 and 142 / 166; 64 over 30,000 88 / 65 and 90 / 67; 1 over 6,000
-// 65 / 43 us. Inserts' neighbour searches stay with k_batch_scan, which leaves a CU's LDS to
-// the queries beside them.)
-bool batch_small_rq(int32_t q, int64_t n, bool uniform);
+// k_batch_scan: where every row's score is kept, up to 45,056 rows for more than 8 results and up to
+// 32,768 for 8 or fewer, whose lists the scan keeps cheaply; and beyond, with one query time and more than
+// 8 results, up to 2^19 rows of 256 and 2^20 of 384 and 512: a tile of narrow rows is little work between
+// two barriers. (The whole call, k_batch_scan / k_batch_rq, one time: 64 queries over 1M rows of 768, 10
+// results, 347 / 323 us; 33 over 150,000 130 / 94; 1 over 1M rows of 256 176 / 193, over 600,000 140 / 132;
+// 33 over 4M rows of 512 761 / 808; 8 results, 33 queries over 600,000 rows of 256 158 / 170, over 2M of 512
+// 414 / 469. Per-query times and decay: 64 over 1M rows of 768 374 / 392.) Inserts' neighbour searches stay
+// with k_batch_scan, which leaves a CU's LDS to the queries beside them.
+bool batch_small_rq(int32_t q, int64_t n, int32_t d, int32_t k, bool uniform);
 // k_batch_rq keeps every row's score (BatchArgs::scores), and the merge selects, where a workgroup would
 // have fewer than kRqFloorTiles tiles: there a floor's passes (rq_sample_rows) and filling and searching
 // lists cost more than a longer merge. (The whole call over rows of 768, one time, lists and floor / scores,

@@ -78,3 +78,15 @@ def test_inserts_keep_to_a_quarter_of_the_chip(so, q):
     for n in ROWS:
         g = check(so._ZN4mars11insert_gridEli(C.c_int64(n), C.c_int32(q)), n, q, 16)
         assert g.n_rranges <= (64 if n <= 2_000_000 else 256), (n, q, g.n_rranges)
+
+
+# up to 64 queries: rows, row length, results, one time
+@pytest.mark.parametrize("q,n,d,k,uniform,rq", [
+    (64, 45_056, 768, 16, False, True), (64, 45_057, 768, 16, False, False), (1, 32_768, 256, 8, False, True),
+    (1, 32_769, 256, 8, True, False), (64, 1_000_000, 768, 8, True, False), (64, 13_000_000, 768, 9, True, True),
+    (1, 1 << 19, 256, 10, True, True), (1, (1 << 19) + 1, 256, 10, True, False), (33, 1 << 20, 512, 10, True, True),
+    (33, (1 << 20) + 1, 384, 10, True, False), (65, 1000, 768, 10, True, False)])
+def test_small_batches_take_the_faster_kernel(so, q, n, d, k, uniform, rq):
+    f = so._ZN4mars14batch_small_rqEiliib
+    f.restype = C.c_bool
+    assert f(C.c_int32(q), C.c_int64(n), C.c_int32(d), C.c_int32(k), C.c_bool(uniform)) == rq
