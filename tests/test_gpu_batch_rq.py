@@ -4,11 +4,9 @@ registers, 16-row tiles through LDS, a sampled score floor).
 - against the fp32 oracle's top-K (the bar of tests/parity.py: scores within 2e-3 of the
   scale, id sets equal up to near-ties) at every supported width, both list sizes, with
   and without a modality filter, one or per-query times, ragged row counts;
-- bit for bit against k_batch_scan, which computes the same MFMA products in the same order: on
-  more rows than are kept whole (45,056), batches of up to 64 queries with per-query times take
-  it, and with one time k_batch_rq; batches of 32 of fewer rows or one time are k_batch_rq's
-  form for up to 64 queries, against its 128- and 256-query forms;
-- floors, lists, tiles with many and few passing rows, and the form that keeps every row;
+- bit for bit against k_batch_scan, which computes the same MFMA products in the same order:
+  mars_query_batch_static in blocks of 32 queries always takes it (scan_batch below);
+- floors, lists, tiles with many and few passing rows, and the form that keeps every row's score;
 - the neighbour-search form (plain dot products, the node itself excluded) against the
   exact CPU k-NN;
 - the merge of the ranges' keys.
@@ -42,6 +40,11 @@ def static_batch(dg, qs, tq, cfg, uniform, block=None):
     return np.concatenate([o[0] for o in out]), np.concatenate([o[1] for o in out])
 
 
+def scan_batch(dg, qs, tq, cfg, uniform):
+    """The same queries by k_batch_scan (no floor; uniform: one decay weight per row)."""
+    return static_batch(dg, qs, tq, cfg, uniform, 32)
+
+
 @pytest.mark.parametrize("d,q,k,filt,uniform", [(256, 129, 5, -1, True), (384, 200, 16, 1, False),
                                                  (512, 256, 8, 2, True), (768, 300, 10, -1, False),
                                                  (768, 520, 16, 0, True), (256, 1000, 3, -1, True),
@@ -71,13 +74,12 @@ def test_rq_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
     buf = mars_amd.DeviceBuffer.from_array(qs)
     try:
         ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # k_batch_rq
-        parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, 32, tq[j:j + 32], cfg)
-                 for j in range(0, q, 32)]
+        want_ids, want_sc = scan_batch(dev.dg, qs, tq, cfg, uniform)
     finally:
         buf.free()
         dev.close()
-    np.testing.assert_array_equal(ids, np.concatenate([p[0] for p in parts]))
-    np.testing.assert_array_equal(sc, np.concatenate([p[1] for p in parts]))
+    np.testing.assert_array_equal(ids, want_ids)
+    np.testing.assert_array_equal(sc.view(np.uint32), want_sc.view(np.uint32))
 
 
 def test_rq_sampled_floor(rng):
@@ -102,8 +104,8 @@ def test_rq_sampled_floor(rng):
 def test_rq_sampled_floor_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
     """The sampled floor drops no row that belongs in a list: on 200K rows (each 256-query
     group's ranges sampled for the floor), the batch's ids and score bits equal those of
-    the same queries scored in batches of 32 (k_batch_scan, which takes no floor, with per-query times), with a modality
-    filter and with per-query times too."""
+    the same queries scored by k_batch_scan, which takes no floor, with a modality filter and
+    with per-query times too."""
     n, d = 200_000, 256
     emb = rng.standard_normal((n, d)).astype(np.float32)
     emb /= np.linalg.norm(emb, axis=1, keepdims=True)
@@ -116,13 +118,12 @@ def test_rq_sampled_floor_equals_scan_bit_for_bit(q, k, filt, uniform, rng):
     buf = mars_amd.DeviceBuffer.from_array(qs)
     try:
         ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # sampled floor
-        parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, min(32, q - j), tq[j:j + 32], cfg)
-                 for j in range(0, q, 32)]
+        want_ids, want_sc = scan_batch(dev.dg, qs, tq, cfg, uniform)
     finally:
         buf.free()
         dev.close()
-    np.testing.assert_array_equal(ids, np.concatenate([p[0] for p in parts]))
-    np.testing.assert_array_equal(sc.view(np.uint32), np.concatenate([p[1] for p in parts]).view(np.uint32))
+    np.testing.assert_array_equal(ids, want_ids)
+    np.testing.assert_array_equal(sc.view(np.uint32), want_sc.view(np.uint32))
 
 
 def test_rq_sampled_floor_sparse_filter_and_neighbours(rng):
@@ -173,15 +174,15 @@ def test_rq_neighbour_search(rng):
     assert np.all(got != np.arange(100, 400)[:, None])
 
 
-# below 12 tiles for each of 256 workgroups every row's key is kept (10 rows to 45,056); from there
-# on a floor and lists
+# below 12 tiles for each of 256 workgroups every row's score is kept (10 rows to 45,056); from there
+# on a floor and lists; 30 and 64 queries: the form of 64 per workgroup
 @pytest.mark.parametrize("n", [10, 41, 4097, 12_289, 11 * 4096, 11 * 4096 + 1, 50_000])
 @pytest.mark.parametrize("q,k,lam,uniform", [(70, 8, LAM, False), (130, 16, LAM, True), (256, 9, 0.0, False),
-                                             (100, 16, -1e-3, False)])
-def test_rq_floors_and_queues_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng):
+                                             (100, 16, -1e-3, False), (30, 7, LAM, True), (64, 16, LAM, True)])
+def test_rq_floors_and_lists_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng):
     """Rows that improve along every range (the sampled first tiles give weak floors, so tiles
-    go through the dense way, the queues and their drains in turn), 40 copies of one row (ties
-    across ranges), rows of zeros and one NaN row: ids and score bits equal k_batch_scan's."""
+    go through the dense and the sparse way in turn), 40 copies of one row (ties across ranges),
+    rows of zeros and one NaN row: ids and score bits equal k_batch_scan's."""
     d = 256
     emb = rng.standard_normal((n, d)).astype(np.float32)
     emb /= np.linalg.norm(emb, axis=1, keepdims=True)
@@ -201,13 +202,12 @@ def test_rq_floors_and_queues_equal_scan_bit_for_bit(n, q, k, lam, uniform, rng)
     buf = mars_amd.DeviceBuffer.from_array(qs)
     try:
         ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)                  # k_batch_rq
-        parts = [mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr + j * d * 4, min(32, q - j), tq[j:j + 32], cfg)
-                 for j in range(0, q, 32)]
+        want_ids, want_sc = scan_batch(dev.dg, qs, tq, cfg, uniform)
     finally:
         buf.free()
         dev.close()
-    np.testing.assert_array_equal(ids, np.concatenate([p[0] for p in parts]))
-    np.testing.assert_array_equal(sc.view(np.uint32), np.concatenate([p[1] for p in parts]).view(np.uint32))
+    np.testing.assert_array_equal(ids, want_ids)
+    np.testing.assert_array_equal(sc.view(np.uint32), want_sc.view(np.uint32))
 
 
 # one merge wave's 512 keys (32 ranges of 16, 64 of 8), more lists, ragged ones
@@ -236,10 +236,10 @@ def test_merge_of_few_and_many_keys(n, q, k, rng):
 
 
 @pytest.mark.parametrize("d", [256, 768])
-@pytest.mark.parametrize("q,k,filt", [(1, 8, -1), (15, 16, 1), (17, 3, -1), (63, 10, 2)])
+@pytest.mark.parametrize("q,k,filt", [(1, 9, -1), (15, 16, 1), (17, 13, -1), (63, 10, 2)])
 def test_small_uniform_batch_equals_scan_bit_for_bit(d, q, k, filt, rng):
-    """Up to 64 queries of one time take k_batch_rq; with one more query of another time the batch
-    takes k_batch_scan (50,000 rows: more than are kept whole). Same ids and score bits."""
+    """Up to 64 queries of one time take k_batch_rq for more than 8 results; with one more query of another
+    time the batch takes k_batch_scan (50,000 rows: more than are kept whole). Same ids and score bits."""
     n = 50_000
     emb, mods, ts, _, _, _ = random_graph(rng, n, d)
     emb[100:130] = emb[100]
@@ -313,3 +313,28 @@ def test_static_short_ranges_equal_scan_bit_for_bit(q, n, k, uniform, rng):
         dev.close()
     np.testing.assert_array_equal(ids, ids2)
     np.testing.assert_array_equal(sc.view(np.uint32), sc2.view(np.uint32))
+
+
+# of more scores than are kept: ranges of 3 tiles (lists without a floor) and of 6 (with one)
+@pytest.mark.parametrize("q,n,k,uniform", [(34_000, 380, 5, False), (34_000, 380, 16, True), (20_000, 700, 7, True),
+                                           (20_000, 700, 12, False)])
+def test_very_large_batches_of_few_rows(q, n, k, uniform, rng):
+    """A batch too large for every row's score keeps lists in short ranges: ids and score bits of a part
+    of its queries equal k_batch_scan's."""
+    emb, mods, ts, _, _, _ = random_graph(rng, n, 256)
+    emb[50:70] = emb[50]
+    emb[n - 3, 1] = np.nan
+    dev = Dev(emb, mods, ts, None, None, fp16=True)
+    qs = emb[rng.integers(0, n - 3, q)]
+    tq = np.full(q, T_Q, np.float32) if uniform else rng.uniform(300, 600, q).astype(np.float32)
+    cfg = RetrievalConfig(top_k=k, time_decay_lambda=LAM, modality_filter=-1 if uniform else 2)
+    buf = mars_amd.DeviceBuffer.from_array(np.ascontiguousarray(qs))
+    try:
+        ids, sc = mars_amd.query_batch(dev.dg, dev.ctx, buf.ptr, q, tq, cfg)
+        part = np.unique(np.r_[0:256, rng.choice(q, 1000), q - 100:q])
+        want_ids, want_sc = scan_batch(dev.dg, qs[part], tq[part], cfg, uniform)
+    finally:
+        buf.free()
+        dev.close()
+    np.testing.assert_array_equal(ids[part], want_ids)
+    np.testing.assert_array_equal(sc[part].view(np.uint32), want_sc.view(np.uint32))

@@ -278,10 +278,10 @@ def test_batch_tiled_widths(d, k, filt, uniform, rng):
                                                    (110_000, 4, -1, False, 0.0), (110_000, 8, 2, True, LAM),
                                                    (110_000, 16, -1, False, LAM)])
 def test_batch_tiled_long_ranges(n, k, filt, uniform, lam, rng):
-    """Batches of 1,030 fused-score queries over long row ranges (k_batch_rq): 60,000 rows
-    without the sampled pass, 110,000 rows with it (its floors drop rows from the first
-    tile on); decay per query and per batch, no decay, filters. A quarter of the queries
-    and the six of the last, partial query group are checked against the oracle's top-K."""
+    """Batches of 1,030 fused-score queries over long row ranges (k_batch_rq) of 60,000 and
+    110,000 rows, with floors from the sampled pass (they drop rows from the first tile on); decay
+    per query and per batch, no decay, filters. A quarter of the queries and the six of the last,
+    partial query group are checked against the oracle's top-K."""
     d, q = 256, 1030
     emb, mods, ts, row, col, _ = random_graph(rng, n, d)
     dev = Dev(emb, mods, ts, row, col, fp16=True)
@@ -302,24 +302,24 @@ def test_batch_tiled_long_ranges(n, k, filt, uniform, lam, rng):
 @pytest.mark.parametrize("d", [256, 384, 512])
 def test_knn_tiled_widths(d, rng):
     """The k-NN builder (plain dot products, the node itself excluded) at the other widths
-    against the exact CPU k-NN: the first 1,024 nodes through k_batch_mm, the other 476
+    against the exact CPU k-NN: all 1,500 nodes in one k_batch_mm launch, the last 476 again
     through k_batch_rq; differing neighbours must be near-ties with the 8th."""
     n = 1500
     emb, mods, ts, _, _, _ = random_graph(rng, n, d)
     dev = Dev(emb, mods, ts, None, None, fp16=True)
     try:
-        got = mars_amd.graph_knn(dev.dg, 8)
         want, sims = corpus.knn_cpu(emb, 8)
         s = emb @ emb.T
         np.fill_diagonal(s, -np.inf)
-        mism = 0
-        for i in range(n):
-            if not np.array_equal(got[i], want[i]):
-                mism += 1
-                for j in set(got[i].tolist()) ^ set(want[i].tolist()):
-                    assert abs(s[i, j] - sims[i, 7]) <= 1e-3, (i, j)
-        assert mism <= 0.02 * n
-        assert np.all(got != np.arange(n)[:, None])
+        for first, got in ((0, mars_amd.graph_knn(dev.dg, 8)), (1024, mars_amd.graph_knn_range(dev.dg, 8, 1024, 476))):
+            mism = 0
+            for i, g in enumerate(got, first):
+                if not np.array_equal(g, want[i]):
+                    mism += 1
+                    for j in set(g.tolist()) ^ set(want[i].tolist()):
+                        assert abs(s[i, j] - sims[i, 7]) <= 1e-3, (i, j)
+            assert mism <= 0.02 * len(got)
+            assert np.all(got != np.arange(first, n)[:, None])
     finally:
         dev.close()
 
