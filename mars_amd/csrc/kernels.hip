@@ -288,7 +288,11 @@ __device__ int bfs_lds(FinShared& sh, const FinalizeArgs& a, int ns, int* levels
     constexpr int R = 4;                       // 1024-edge rounds cached in registers
     const int tid = int(threadIdx.x);
     for (int i = tid; i < kHashCap; i += kFinThreads) { sh.u.bfs.hkey[i] = 0u; sh.u.bfs.hval[i] = 0xFFFFFFFFu; }
-    if (tid == 0) { sh.s_misc[4] = 0; sh.s_misc[5] = 0; sh.bound = bthr; }   // wave 0's: the seeds' rk-th
+    if (tid == 0) {
+        sh.s_misc[4] = 0;
+        sh.s_misc[5] = 0;
+        if constexpr (MODE != kBfsUnscored) sh.bound = bthr;   // wave 0's: the seeds' rk-th
+    }
     __syncthreads();
     if (tid < ns) {
         const int slot = hash_find_or_insert(sh, sh.seed_id[tid]);
