@@ -190,7 +190,8 @@ int mars_graph_set_csr(mars_graph* g, int32_t num_edges, const int32_t* row_offs
  * src/cmng_build.cu:135-245). Each node's list is certified exact when its k-th exact
  * score beats the 16th candidate's fp16 score by more than the fp16 scan's error bound
  * (from the fp16 copy's row-norm maxima); the lists the certificate does not cover are
- * found again by exact fp32 scans (mars_graph_knn_report counts both). */
+ * found again by exact fp32 scans (mars_graph_knn_report counts both). The graph keeps
+ * up to 64 MiB of device scratch and 4 MiB of pinned memory for the next build. */
 int mars_graph_knn(mars_graph* g, int32_t k, int32_t* nbrs);
 /* Counts of the last k-NN builder call on g (mars_graph_knn, _blocked, _blocks, _range):
  * the nodes whose lists the certificate did not cover, and of those the nodes found again

@@ -23,7 +23,7 @@
 //  against its query's bound (a floor from the sampled pass of launch_batch_topk, then its K-th
 //  best), between the MFMAs of the next tile; the few that reach it are fused, exactly as
 //  k_batch_scan does, and offered to their query's list of K keys. Output: K keys per (query,
-//  row range), the layout k_batch_merge reads.
+//  row range), or over few rows every row's score (BatchArgs::scores), as k_batch_merge reads them.
 //
 //  What bounds it (1M rows, d = 768, 256 queries of one time): the pass takes 375 us, 360 us with
 //  the selection switched off, against 160 us of MFMAs alone and 260 us of row loads alone: the

@@ -567,7 +567,7 @@ bool batch_dim_supported(int32_t d);
 //   Q > kRqMaxScanQ               k_batch_rq (batch_rq.hip): the queries held in registers
 //                                 (64, 128 or 256 per workgroup, batch_rq_tiles x 16 per wave),
 //                                 16-row tiles streamed through LDS, a sampled score floor
-//                                 (Q = 256: full pass 375-390 us)
+//                                 (Q = 256: full pass 375-406 us over several boxes)
 //   neighbour searches, Q >= kGemmMinQ
 //                                 k_batch_mm: 256-query x 256-row LDS tiles, thresholds from
 //                                 the sampled floor (chunks of 1024 queries 1.90 ms, against 2.86
